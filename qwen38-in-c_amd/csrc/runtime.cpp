@@ -519,12 +519,79 @@ int run_gemv_group(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
     return Q35MM_OK;
 }
 
-// Weights sharing K, in groups of up to 8 tokens; stream-K weights share one
-// launch, row-split weights another.
+// Batched decode of row-split weights (gemv_batch.hip): m > kGemvMaxM tokens
+// in passes of up to kBatchTokens (bounds the workspace).  pair: w is gate
+// and up of one shape and dY[0] receives silu(gate) * up.  Returns kNoRoom,
+// with nothing launched, when there is no scratch for it -- a capture on a
+// stream without a set of its own (scr null) or with too small a one, or the
+// fixed scratch of an allocation-free call -- and the caller takes the
+// launches of eight tokens, which need none and give the same bits.
+constexpr uint32_t kBatchTokens = 64;
+constexpr int kNoRoom = -1001;   // internal
+
+int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const float *dX, float *const *dY,
+                   hipStream_t st, float *const *resid, Scratch *scr, bool pair) {
+    Scratch &sc = scr ? *scr : scratch_for(st);
+    if (!scr && sc.capturing && !g_dev.scratch.count(st)) return kNoRoom;
+    const uint32_t cols = w[0]->w.cols, kb = w[0]->w.kb, mp = std::min(m, kBatchTokens);
+    uint32_t groups = 0, wsoff = 0;
+    BatchParams p{};
+    p.kb = kb;
+    p.nseg = nseg;
+    p.nr = g_dev.rows_waves;
+    for (uint32_t s = 0; s < nseg; s++) groups += w[s]->w.nb;
+    // A workgroup per row group and token tile where that gives every CU one;
+    // otherwise one per K range too, their sums added by a second kernel.
+    bool seq = pair || groups * ((mp + batch_tile(mp) - 1) / batch_tile(mp)) >= g_dev.cus;
+    for (uint32_t s = 0; s < nseg; s++) {
+        const Weight &ws = w[s]->w;
+        GemvSeg &g = p.seg[s];
+        g.codes = ws.codes;
+        g.scale = ws.scale;
+        g.rows = ws.rows;
+        g.ldy = ws.rows;
+        g.nb = ws.nb;
+        g.ws_off = wsoff;
+        wsoff += p.nr * mp * ws.nb * kBlock;
+    }
+    const size_t xb = (batch_act_bytes(mp, kb) + 255) & ~(size_t)255;
+    size_t wsb = (size_t)wsoff * sizeof(float);
+    if (sc.fixed && xb + wsb > kNoAllocBytes) seq = true;
+    if (seq) wsb = 0;
+    if (sc.fixed ? xb + wsb > kNoAllocBytes : sc.capturing && (sc.xb.cap < xb || sc.ws.cap < wsb)) return kNoRoom;
+    uint16_t *xs = nullptr;
+    const int rc = scratch_gemm(sc, xb, wsb, &xs, &p.ws);
+    if (rc) return rc;
+    p.xs = reinterpret_cast<const uint8_t *>(xs);
+    const bool vec = aligned16(dX) && cols % 8 == 0;
+    for (uint32_t t0 = 0; t0 < m; t0 += mp) {
+        p.m = std::min(mp, m - t0);
+        const uint32_t T = batch_tile(p.m);
+        float *xf = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(xs) +
+                                              (size_t)((p.m + T - 1) / T) * kb * 768 * T);
+        p.xf = xf;
+        for (uint32_t s = 0; s < nseg; s++) {
+            const size_t o = (size_t)t0 * p.seg[s].ldy;
+            p.seg[s].y = dY[pair ? 0 : s] + o;
+            p.seg[s].resid = resid ? resid[s] + o : nullptr;
+        }
+        HIP_TRY(launch_split_act(dX + (size_t)t0 * cols, cols, p.m, cols, kb, vec, reinterpret_cast<uint8_t *>(xs), xf, st));
+        HIP_TRY(launch_gemv_batch(p, seq, pair, st));
+    }
+    return Q35MM_OK;
+}
+
+// Weights sharing K: more than eight tokens of row-split weights as one
+// batch, everything else in groups of up to eight tokens; stream-K weights
+// share one launch, row-split weights another.
 int run_gemv(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const float *dX,
              float *const *dY, hipStream_t st, const GemvInput &in = GemvInput(),
              float *const *resid = nullptr, Scratch *scr = nullptr) {
     const uint32_t cols = w[0]->w.cols;
+    if (m > kGemvMaxM && in.xmode == kXPlain && uses_gemv_rows(w[0]->w)) {   // same K: one kind for all
+        const int rc = run_gemv_batch(w, nseg, m, dX, dY, st, resid, scr, false);
+        if (rc != kNoRoom) return rc;
+    }
     for (uint32_t t0 = 0; t0 < m; t0 += kGemvMaxM) {
         const uint32_t mg = std::min(kGemvMaxM, m - t0);
         GemvInput ig = in;
@@ -1738,13 +1805,16 @@ Q35MM_API int q35mm_mlp(const q35mm_weight *gate, const q35mm_weight *up, const 
             // residual add.
             const bool norm_in = m == 1 && H <= kPairNormMaxCols && g_dev.mlp_pair == 1;
             if (!norm_in) HIP_TRY(launch_rmsnorm(dX, H, dNormW, xn, H, m, H, eps, st));
-            for (uint32_t t0 = 0; t0 < m; t0 += kGemvMaxM) {
+            const q35mm_weight *gu[2] = {gate, up};
+            rc = m > kGemvMaxM ? run_gemv_batch(gu, 2, m, xn, &g, st, nullptr, &scr, true) : kNoRoom;
+            if (rc && rc != kNoRoom) return rc;
+            for (uint32_t t0 = 0; rc == kNoRoom && t0 < m; t0 += kGemvMaxM) {
                 const uint32_t mt = std::min(kGemvMaxM, m - t0);
-                rc = run_mlp_pair(gate, up, mt, (norm_in ? dX : xn) + (size_t)t0 * H, norm_in ? dNormW : nullptr, eps,
-                                  g + (size_t)t0 * I, st);
-                if (rc) return rc;
+                const int e = run_mlp_pair(gate, up, mt, (norm_in ? dX : xn) + (size_t)t0 * H,
+                                           norm_in ? dNormW : nullptr, eps, g + (size_t)t0 * I, st);
+                if (e) return e;
             }
-            return run_gemv(dn, 1, m, g, dy, st, GemvInput(), dy);
+            return run_gemv(dn, 1, m, g, dy, st, GemvInput(), dy, &scr);
         }
         const bool fuse_norm = !g_dev.mlp_unfused && gemv_norm_fits(mg, H) && !uses_gemv_rows(gate->w) &&
                                !uses_gemv_rows(up->w);

@@ -1,0 +1,132 @@
+"""Batched decode (gemv_batch.hip): more than eight tokens of a row-split
+weight in one pass over it, below the prefill GEMM.
+
+Its sums are the row-split GEMV's, so every row of a batch is, bit for bit,
+the row of a call of one to eight tokens (which the other tests hold against
+the oracle): edges of the token tiles (16 and 32), 4..160 K blocks (a last
+turn of the three-deep ring of each length), partial blocks both ways, both
+work splits (few and many row groups), several weights, values of any
+magnitude.
+"""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows_of_small_calls(q, ws, X, gpu):
+    import torch
+    Ys = [torch.empty((X.shape[0], w.rows), device=gpu) for w in ws]
+    for t in range(0, X.shape[0], 8):
+        part = [torch.empty((min(8, X.shape[0] - t), w.rows), device=gpu) for w in ws]
+        q.matmul_multi(ws, X[t:t + 8].clone(), part)
+        for Y, p in zip(Ys, part):
+            Y[t:t + 8] = p
+    return Ys
+
+
+def _same_bits(a, b):
+    import torch
+    assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+
+
+@pytest.mark.parametrize("m,k,rows", [(9, 400, (200,)), (16, 1003, (4100,)), (17, 5120, (1024,)), (32, 640, (33000,)),
+                                      (33, 20480, (129,)), (63, 17400, (300,)), (24, 1032, (130, 48, 1, 5000)),
+                                      (12, 897, (20000, 16000)), (63, 768, (16300, 70)), (10, 512, (1,))])
+def test_batch_rows_are_small_calls_bitwise(q, wl, gpu, m, k, rows):
+    import torch
+    ws = [q.Weight(*wl.gen_weight_ragged(k + i, n, k)) for i, n in enumerate(rows)]
+    X = torch.from_numpy(wl.gen_act(m, m, k, outlier_frac=0.01)).to(gpu)
+    Ys = [torch.empty((m, n), device=gpu) for n in rows]
+    q.matmul_multi(ws, X, Ys)
+    for Y, R in zip(Ys, _rows_of_small_calls(q, ws, X, gpu)):
+        _same_bits(Y, R)
+    big = torch.zeros(m * k + 1, device=gpu)   # rows 4 bytes past a 16-byte boundary
+    big[1:] = X.reshape(-1)
+    Y1 = torch.empty_like(Ys[0])
+    q.matmul(ws[0], big[1:].view(m, k), Y1)
+    _same_bits(Y1, Ys[0])
+    Y2 = torch.empty_like(Ys[0])
+    q.matmul_noalloc(ws[0], X, Y2)
+    _same_bits(Y2, Ys[0])
+    for w in ws:
+        w.free()
+
+
+@pytest.mark.parametrize("m", [16, 40])
+def test_batch_wide_values(q, wl, gpu, m):
+    """Blocks holding values past 2^96 or infinities are staged shifted."""
+    import torch
+    k, n = 1000, 300
+    w = q.Weight(*wl.gen_weight(5, n, k))
+    X = wl.gen_act(6, m, k)
+    X[0, 3], X[1, 700], X[2, 999] = np.inf, -np.inf, np.float32(3.4e38)
+    X[m - 1, 130], X[5, 131] = np.float32(-2e30), np.nan
+    X = torch.from_numpy(X).to(gpu)
+    Y = torch.empty((m, n), device=gpu)
+    q.matmul(w, X, Y)
+    R = _rows_of_small_calls(q, [w], X, gpu)[0]
+    assert torch.equal(Y.isnan(), R.isnan())
+    _same_bits(Y.nan_to_num(nan=0.0, posinf=np.inf, neginf=-np.inf), R.nan_to_num(nan=0.0, posinf=np.inf, neginf=-np.inf))
+    w.free()
+
+
+@pytest.mark.parametrize("m,H,I", [(9, 640, 1664), (16, 1032, 4100), (31, 5120, 1000), (63, 512, 16400)])
+def test_batch_mlp_is_small_calls_bitwise(q, wl, gpu, m, H, I):
+    """Gate and up in one pass forming silu(gate) * up; residual added."""
+    import torch
+    w = [q.Weight(*wl.gen_weight(H + i, *s)) for i, s in enumerate(((I, H), (I, H), (H, I)))]
+    rng = np.random.default_rng(m)
+    nw = torch.from_numpy((rng.standard_normal(H) * 0.1).astype(np.float32)).to(gpu)
+    X = torch.from_numpy(rng.standard_normal((m, H)).astype(np.float32)).to(gpu)
+    R = X.clone()
+    for t in range(0, m, 8):
+        part = R[t:t + 8].clone()
+        q.mlp(*w, nw, part)
+        R[t:t + 8] = part
+    q.mlp(*w, nw, X)
+    _same_bits(X, R)
+    for x in w:
+        x.free()
+
+
+def test_batch_beyond_the_gemm(q, wl, gpu):
+    """Block scales too far apart for the prefill GEMM: any m on this path,
+    in passes of 64 tokens."""
+    import torch
+    W, sc = wl.gen_weight(9, 260, 768)
+    sc = sc.copy()
+    sc[0, 0], sc[0, 1] = 0x6F80, 0x3380     # 2^96 and 2^-24
+    w = q.Weight(W, sc)
+    X = torch.from_numpy(wl.gen_act(3, 150, 768)).to(gpu)
+    Y = torch.empty((150, 260), device=gpu)
+    q.matmul(w, X, Y)
+    _same_bits(Y, _rows_of_small_calls(q, [w], X, gpu)[0])
+    w.free()
+
+
+def test_batch_capture(q, wl, gpu):
+    """A capture on a stream that has no scratch yet and one after a call of
+    the same size on that stream both replay to the eager bits."""
+    import torch
+    w = q.Weight(*wl.gen_weight(12, 700, 1024))
+    X = torch.from_numpy(wl.gen_act(13, 24, 1024)).to(gpu)
+    want = _rows_of_small_calls(q, [w], X, gpu)[0]
+    for warm in (False, True):
+        s = torch.cuda.Stream()
+        Y = torch.zeros((24, 700), device=gpu)
+        torch.cuda.synchronize()
+        if warm:
+            with torch.cuda.stream(s):
+                q.matmul(w, X, Y)
+            torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            q.matmul(w, X, Y)
+        for _ in range(3):
+            Y.zero_()
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            _same_bits(Y, want)
+    w.free()
