@@ -41,22 +41,33 @@ namespace {
 
 typedef __attribute__((address_space(3))) uint8_t lds_u8;
 
-constexpr uint32_t kRing = 3;        // K blocks of activations in LDS, of weights in registers
-constexpr uint32_t kWLoads = 4;      // 1 KiB weight loads per wavefront and K block
+// A stage is 12 KiB of split activations: half a K block at 32 tokens, a
+// whole one at 16.
+constexpr uint32_t kRing = 4;        // stages of activations in LDS, of weights in registers
+constexpr uint32_t kPieces = 3;      // 1 KiB activation copies per wavefront and stage
 
-// Per K block: 8 MFMA steps (chunk j < 4, half q < 2) of 3 T rows x 2 x 16
-// bytes: step (j, q), h = lane / 32, part, token at
-// ((((j*2 + q) * 2 + h) * 3 + part) * T + token) * 16.
+// Per K block: 8 MFMA steps (chunk j < 4, half q < 2), each an MFMA's A
+// operand after another as its lanes read them (lane * 16: consecutive, or
+// the two halves of a wavefront meet in the same LDS banks):
+//   T = 32: one operand per part, rows = tokens
+//   T = 16: parts 0 and 1 (rows 16 part + token), then part 2 (16 rows)
+// part_off gives the place of (h = lane / 32, part, token) in a step.
 template <uint32_t T>
 struct BatchGeo {
-    static constexpr uint32_t kHalf = 48 * T;         // one h of a step
-    static constexpr uint32_t kStep = 2 * kHalf;
-    static constexpr uint32_t kStage = 8 * kStep;     // 12 or 24 KiB
-    static constexpr uint32_t kPieces = kStage / kChunkBytes / 4;   // 1 KiB copies per wavefront
+    static constexpr uint32_t kStep = 3 * T * 2 * 16;
+    static constexpr uint32_t kBlk = 8 * kStep;       // one K block
+    static constexpr uint32_t kStages = T / 16;       // per K block
+    static constexpr uint32_t kStage = kBlk / kStages;
+    static constexpr uint32_t kChunks = 4 / kStages;  // 32-column chunks (1 KiB weight loads) per stage
     // MFMAs per step: 32 A rows hold one part of 32 tokens, or parts 0 and 1
     // of 16 tokens and, in a second MFMA, part 2
     static constexpr uint32_t kOps = T == 32 ? 3 : 2;
     static constexpr uint32_t kRegs = T / 2;          // token rows per lane and part
+    static_assert(kStage == 4 * kPieces * kChunkBytes, "four wavefronts copy a stage");
+    static __device__ __forceinline__ uint32_t part_off(uint32_t h, uint32_t part, uint32_t t) {
+        if constexpr (T == 32) return part * 1024 + h * 512 + t * 16;
+        return part < 2 ? h * 512 + part * 256 + t * 16 : 1024 + h * 256 + t * 16;
+    }
 };
 
 // One wavefront copies 1 KiB to LDS: lane l's 16 bytes at base + soff + voff
@@ -75,70 +86,109 @@ constexpr uint32_t wait_vm_lgkm0(uint32_t n) { return (n & 15u) | ((n >> 4) << 1
 
 }  // namespace
 
+// Eight columns of a token, split (shifted first if the block is wide), to
+// the three parts' places in unit u of the K block at blk (columns 8u..8u+7).
+template <uint32_t T>
+__device__ __forceinline__ void store_split(uint8_t *blk, uint32_t u, uint32_t t, const float (&v)[8], bool wide) {
+    using Geo = BatchGeo<T>;
+    const uint32_t j = u >> 2, h = (u >> 1) & 1, q = u & 1;   // columns 32 j + 16 h + 8 q
+    uint32_t p0[4], p1[4], p2[4];
+#pragma unroll
+    for (uint32_t e = 0; e < 4; e++) {
+        if (__builtin_expect(wide, 0)) {
+            split3_bf16x2(v[2 * e] * kActShift, v[2 * e + 1] * kActShift, p0[e], p1[e], p2[e]);
+            split3_fix_inf(p0[e], p1[e], p2[e]);
+        } else {
+            split3_bf16x2(v[2 * e], v[2 * e + 1], p0[e], p1[e], p2[e]);
+        }
+    }
+    uint8_t *const d = blk + (j * 2 + q) * Geo::kStep;
+    *reinterpret_cast<u32x4_t *>(d + Geo::part_off(h, 0, t)) = u32x4_t{p0[0], p0[1], p0[2], p0[3]};
+    *reinterpret_cast<u32x4_t *>(d + Geo::part_off(h, 1, t)) = u32x4_t{p1[0], p1[1], p1[2], p1[3]};
+    *reinterpret_cast<u32x4_t *>(d + Geo::part_off(h, 2, t)) = u32x4_t{p2[0], p2[1], p2[2], p2[3]};
+}
+
 // X fp32 [m][ldx] -> split A operands (BatchGeo's layout per token tile and
 // K block) and one scale factor per tile and K block: 1, or kActUnshift for a
 // block that holds a wide value and was staged times kActShift.  Tokens past
 // m and columns past k are zeros.  One workgroup per tile and K block; a
 // thread splits eight columns of a token.
 template <uint32_t T, bool VEC>
-__global__ __launch_bounds__(256) void split_act_kernel(const float *__restrict__ x, uint32_t ldx, uint32_t m,
-                                                        uint32_t k, uint32_t kb_total, uint8_t *__restrict__ xs,
-                                                        float *__restrict__ xf) {
-    using Geo = BatchGeo<T>;
-    constexpr uint32_t N = T * 16 / 256;
+__global__ __launch_bounds__(16 * T) void split_act_kernel(const float *__restrict__ x, uint32_t ldx, uint32_t m,
+                                                           uint32_t k, uint32_t kb_total, uint8_t *__restrict__ xs,
+                                                           float *__restrict__ xf) {
     const uint32_t kb = blockIdx.x % kb_total, tile = blockIdx.x / kb_total;
-    float v[N][8];
+    const uint32_t tt = threadIdx.x % T, u = threadIdx.x / T, t = tile * T + tt, c = kb * kBlock + u * 8;
+    const float *row = x + (size_t)min(t, m - 1) * ldx;
+    float v[8];
+    if constexpr (VEC) {   // rows 16-byte aligned, k % 8 == 0
+        const float4 a = *reinterpret_cast<const float4 *>(row + min(c, k - 8));
+        const float4 b = *reinterpret_cast<const float4 *>(row + min(c, k - 8) + 4);
+        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+        v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else {
 #pragma unroll
-    for (uint32_t i = 0; i < N; i++) {
-        const uint32_t idx = threadIdx.x + 256 * i, t = tile * T + idx % T, c = kb * kBlock + (idx / T) * 8;
-        const float *row = x + (size_t)min(t, m - 1) * ldx;
-        if constexpr (VEC) {   // rows 16-byte aligned, k % 8 == 0
-            const float4 a = *reinterpret_cast<const float4 *>(row + min(c, k - 8));
-            const float4 b = *reinterpret_cast<const float4 *>(row + min(c, k - 8) + 4);
-            v[i][0] = a.x; v[i][1] = a.y; v[i][2] = a.z; v[i][3] = a.w;
-            v[i][4] = b.x; v[i][5] = b.y; v[i][6] = b.z; v[i][7] = b.w;
-        } else {
-#pragma unroll
-            for (uint32_t e = 0; e < 8; e++) v[i][e] = row[min(c + e, k - 1)];
-        }
-#pragma unroll
-        for (uint32_t e = 0; e < 8; e++)
-            if (t >= m || c + e >= k) v[i][e] = 0.0f;
+        for (uint32_t e = 0; e < 8; e++) v[e] = row[min(c + e, k - 1)];
     }
-    bool w = false;
 #pragma unroll
-    for (uint32_t i = 0; i < N; i++) w |= max_abs(v[i]) >= kActWide;
-    const bool wide = __syncthreads_or(w) != 0;
+    for (uint32_t e = 0; e < 8; e++)
+        if (t >= m || c + e >= k) v[e] = 0.0f;
+    const bool wide = __syncthreads_or(max_abs(v) >= kActWide) != 0;
     if (threadIdx.x == 0) xf[blockIdx.x] = wide ? kActUnshift : 1.0f;
-    uint8_t *const base = xs + (size_t)blockIdx.x * Geo::kStage;
-#pragma unroll
-    for (uint32_t i = 0; i < N; i++) {
-        const uint32_t idx = threadIdx.x + 256 * i, t = idx % T, u = idx / T;
-        const uint32_t j = u >> 2, h = (u >> 1) & 1, q = u & 1;   // columns 32 j + 16 h + 8 q
-        uint32_t p0[4], p1[4], p2[4];
-#pragma unroll
-        for (uint32_t e = 0; e < 4; e++) {
-            if (__builtin_expect(wide, 0)) {
-                split3_bf16x2(v[i][2 * e] * kActShift, v[i][2 * e + 1] * kActShift, p0[e], p1[e], p2[e]);
-                split3_fix_inf(p0[e], p1[e], p2[e]);
-            } else {
-                split3_bf16x2(v[i][2 * e], v[i][2 * e + 1], p0[e], p1[e], p2[e]);
-            }
-        }
-        u32x4_t *dst = reinterpret_cast<u32x4_t *>(base + (j * 2 + q) * Geo::kStep + h * Geo::kHalf + t * 16);
-        dst[0] = u32x4_t{p0[0], p0[1], p0[2], p0[3]};
-        dst[T] = u32x4_t{p1[0], p1[1], p1[2], p1[3]};
-        dst[2 * T] = u32x4_t{p2[0], p2[1], p2[2], p2[3]};
-    }
+    store_split<T>(xs + (size_t)blockIdx.x * BatchGeo<T>::kBlk, u, tt, v, wide);
 }
 
-// T tokens per workgroup; SEQ: all K ranges in the workgroup, else one of
-// them, its sums to p.ws; PAIR (SEQ only): 64 rows of gate (segment 0) and
-// the same rows of up (segment 1), writing silu(gate) * up.
-template <uint32_t T, bool SEQ, bool PAIR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(T == 16 ? 4 : 2, 8)))
+// silu(gate) * up of the range sums of two weights (segments 0 and 1), split
+// as split_act_kernel splits a stored product: the next weight's activations
+// without its fp32 rows in between.  One workgroup per token tile and K block
+// of the next weight, one thread per token and eight columns, columns fastest
+// (the range sums, 8 x 4 bytes an output, outweigh the 6 written).
+template <uint32_t T, uint32_t NR>
+__global__ __launch_bounds__(16 * T) void batch_swiglu_kernel(BatchParams p, uint32_t kb_total, uint8_t *__restrict__ xs,
+                                                              float *__restrict__ xf) {
+    using Geo = BatchGeo<T>;
+    const uint32_t kb = blockIdx.x % kb_total, tile = blockIdx.x / kb_total;
+    const uint32_t u = threadIdx.x & 15, tt = threadIdx.x >> 4, t = tile * T + tt, c = kb * kBlock + u * 8;
+    const uint32_t rows = p.seg[0].rows;
+    const size_t ld = (size_t)p.seg[0].nb * kBlock;
+    float v[8] = {};
+    if (t < p.m) {
+        // every range's sums are loaded before the first is used: one memory
+        // round trip, not one per range
+        float4 w[2][NR][2];
+#pragma unroll
+        for (uint32_t z = 0; z < 2; z++) {
+            const float *src = p.ws + p.seg[z].ws_off + (size_t)t * ld + c;   // rows padded to whole K blocks
+#pragma unroll
+            for (uint32_t r = 0; r < NR; r++)
+#pragma unroll
+                for (uint32_t i = 0; i < 2; i++)
+                    w[z][r][i] = *reinterpret_cast<const float4 *>(src + (size_t)r * p.m * ld + 4 * i);
+        }
+        float sum[2][8];
+#pragma unroll
+        for (uint32_t z = 0; z < 2; z++)
+#pragma unroll
+            for (uint32_t r = 0; r < NR; r++)
+#pragma unroll
+                for (uint32_t i = 0; i < 2; i++) {
+                    const float4 f = w[z][r][i];
+                    const float q[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+                    for (uint32_t e = 0; e < 4; e++) sum[z][4 * i + e] = r == 0 ? q[e] : sum[z][4 * i + e] + q[e];
+                }
+#pragma unroll
+        for (uint32_t e = 0; e < 8; e++) v[e] = c + e < rows ? swiglu1(sum[0][e], sum[1][e]) : 0.0f;
+    }
+    const bool wide = __syncthreads_or(max_abs(v) >= kActWide) != 0;
+    if (threadIdx.x == 0) xf[blockIdx.x] = wide ? kActUnshift : 1.0f;
+    store_split<T>(xs + (size_t)blockIdx.x * Geo::kBlk, u, tt, v, wide);
+}
+
+// One K range of a 128-row group for T tokens: its sums to p.ws.
+template <uint32_t T, bool STREAM>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8)))
 void gemv_batch_kernel(BatchParams p) {
-    static_assert(SEQ || !PAIR, "paired rows need whole sums");
     using Geo = BatchGeo<T>;
     extern __shared__ __align__(16) uint8_t lds[];
     // block scales (times the shifted blocks' factor), after the ring.  One
@@ -150,125 +200,119 @@ void gemv_batch_kernel(BatchParams p) {
     // workgroups apart, i.e. on one XCD (workgroups go round-robin over 8).
     const uint32_t per = 8 * p.tiles;
     const uint32_t tile = (blockIdx.x % per) / 8, item = blockIdx.x / per * 8 + blockIdx.x % 8;
-    if (item >= p.items) return;
-    const uint32_t grp = SEQ ? item : item % p.groups, range = SEQ ? 0 : item / p.groups;
+    if (item >= p.groups * p.nr) return;
+    const uint32_t grp = item % p.groups, range = item / p.groups;
 
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // 32-row sub-tile
     uint32_t si = 0;
-    if constexpr (PAIR) {
-        si = wv >> 1;
-    } else {
 #pragma unroll
-        for (uint32_t i = 1; i < 4; i++)
-            if (i < p.nseg && grp >= p.seg[i].cta_begin) si = i;
-    }
+    for (uint32_t i = 1; i < 4; i++)
+        if (i < p.nseg && grp >= p.seg[i].cta_begin) si = i;
     const GemvSeg &sg = p.seg[si];
     const uint32_t KB = p.kb, NR = p.nr;
-    // this wavefront's 32-row sub-tile of the segment and its 128-row group
-    const uint32_t sub = PAIR ? grp * 2 + (wv & 1) : (grp - sg.cta_begin) * 4 + wv;
-    const uint32_t rg = sub >> 2;
-    const uint32_t k0 = SEQ ? 0 : range * KB / NR, k1 = SEQ ? KB : (range + 1) * KB / NR, n = k1 - k0;
+    const uint32_t rg = grp - sg.cta_begin;   // 128-row group of the segment
+    const uint32_t k0 = range * KB / NR, n = (range + 1) * KB / NR - k0;
 
     // ---- block scales, loaded before the stream so that waiting for them
     // waits for nothing else ----
-    constexpr uint32_t kTabs = PAIR ? 2 : 1;
-    float sc[kTabs];
-#pragma unroll
-    for (uint32_t z = 0; z < kTabs; z++) {
-        const GemvSeg &ss = PAIR ? p.seg[z] : sg;
-        const uint32_t kb = k0 + min(threadIdx.x, n - 1);
-        sc[z] = ss.scale[(size_t)rg * KB + kb] * p.xf[(size_t)tile * KB + kb];
-    }
+    const uint32_t kbl = k0 + min(threadIdx.x, n - 1);
+    const float sc = sg.scale[(size_t)rg * KB + kbl] * p.xf[(size_t)tile * KB + kbl];
 
-    // ---- weight and activation streams: K block s of the range is waited
-    // for at step s and issued at step s - 2, activations first.  Loads are
-    // unconditional (blocks past the end read the last one again), so the
-    // wait before each step is static: everything but the next block's ----
-    const uint8_t *const codes = sg.codes + ((size_t)rg * KB + k0) * kBlockBytes + (sub & 3) * kSubBytes + lane * 16;
-    const uint8_t *const xsrc = p.xs + ((size_t)tile * KB + k0) * Geo::kStage;
-    const uint32_t xbytes = n * Geo::kStage;
-    const uint32_t xoff = wv * (Geo::kPieces * kChunkBytes);
-    lds_u8 *const ring = (lds_u8 *)lds + wv * (Geo::kPieces * kChunkBytes);
-    u32x4_t wbuf[kRing][kWLoads];
+    // ---- weight and activation streams: stage s is issued, activations
+    // first, at the end of stage s - 4 and waited for at the end of stage
+    // s - 1.  Loads are unconditional (stages past the end read the last one
+    // again), so that wait is static: everything but the two newest ----
+    const uint32_t ns = n * Geo::kStages;
+    const uint8_t *const codes = sg.codes + ((size_t)rg * KB + k0) * kBlockBytes + wv * kSubBytes + lane * 16;
+    const uint8_t *const xsrc = p.xs + ((size_t)tile * KB + k0) * Geo::kBlk;
+    const uint32_t xbytes = n * Geo::kBlk;
+    const uint32_t xoff = wv * (kPieces * kChunkBytes);
+    lds_u8 *const ring = (lds_u8 *)lds + xoff;
+    u32x4_t wbuf[kRing][Geo::kChunks];
     auto issue = [&](uint32_t slot, uint32_t s) {
-        const uint32_t kb = min(s, n - 1);
+        const uint32_t st = min(s, ns - 1);
 #pragma unroll
-        for (uint32_t i = 0; i < Geo::kPieces; i++)
+        for (uint32_t i = 0; i < kPieces; i++)
             copy_1k(xsrc, xbytes, ring + slot * Geo::kStage + i * kChunkBytes, lane * 16,
-                    kb * Geo::kStage + xoff + i * kChunkBytes);
-        const uint8_t *src = codes + (size_t)kb * kBlockBytes;
+                    st * Geo::kStage + xoff + i * kChunkBytes);
+        const uint8_t *src = codes + (size_t)(st / Geo::kStages) * kBlockBytes +
+                             (st % Geo::kStages) * (Geo::kChunks * kChunkBytes);
 #pragma unroll
-        for (uint32_t j = 0; j < kWLoads; j++)
-            wbuf[slot][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(src + j * kChunkBytes));
+        for (uint32_t j = 0; j < Geo::kChunks; j++)
+            if constexpr (STREAM)
+                wbuf[slot][j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t *>(src + j * kChunkBytes));
+            else
+                wbuf[slot][j] = *reinterpret_cast<const u32x4_t *>(src + j * kChunkBytes);
     };
     __builtin_amdgcn_sched_barrier(0);
-    issue(0, 0);
-    issue(1, 1);
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (uint32_t z = 0; z < kTabs; z++)
-        if (threadIdx.x < n) tab[z * kGemvRsMaxKb + threadIdx.x] = sc[z];
+    for (uint32_t d = 0; d < kRing; d++) issue(d, d);
+    __builtin_amdgcn_sched_barrier(0);
+    if (threadIdx.x < n) tab[threadIdx.x] = sc;
 
-    // This lane's A row: a part of a token (T = 32: token = row; T = 16: row
-    // / 16 = part 0 or 1, the second MFMA's rows all part 2)
     const uint32_t hh = lane >> 5, mrow = lane & 31;
-    const uint32_t a0 = hh * Geo::kHalf + mrow * 16;
-    const uint32_t a1 = T == 32 ? a0 + 512 : hh * Geo::kHalf + 512 + (mrow & 15) * 16;
-    const float *const mytab = tab + (PAIR ? si * kGemvRsMaxKb : 0);
+    const uint32_t a0 = lane * 16, a1 = 1024 + (T == 32 ? lane * 16 : hh * 256 + (mrow & 15) * 16);
 
-    f32x16_t acc[Geo::kOps] = {};
+    // Software pipeline of one wavefront.  The MFMAs of step i (its operands
+    // and its bf16 weights in registers) run with, beside each of them, the
+    // LDS read of one operand and two of the conversions of step i + 1 and
+    // the scaling of two or three sums of the previous K block (part is
+    // double): left in one piece after the block's last MFMA, the scaling
+    // and the first reads of a stage cost a lone wavefront half its time.
+    constexpr uint32_t kSteps = 2 * Geo::kChunks;              // per stage
+    constexpr uint32_t kSlots = 8 * Geo::kOps;                 // MFMAs per K block
+    constexpr uint32_t kSums = T == 32 ? 48 : 24;              // acc[e / 16][e % 16], e < kSums
+    f32x16_t acc[Geo::kOps] = {}, part[2][Geo::kOps] = {};
     const f32x16_t zero = {};
-    float tot[Geo::kRegs];
-    // The sum of a finished range, per token row: (part 0 + part 1) + part 2
-    auto range_sum = [&](uint32_t r) {
-        if constexpr (T == 32)
-            return (acc[0][r] + acc[1][r]) + acc[Geo::kOps - 1][r];
-        else
-            return (acc[0][r] + acc[0][r + 8]) + acc[1][r];
+    u32x4_t aop[2][Geo::kOps], bop[2];
+    float sc_prev = 0.0f, sc_cur = 0.0f;
+    auto read_a = [&](uint32_t slot, uint32_t i, uint32_t o) {
+        aop[i & 1][o] = *reinterpret_cast<const u32x4_t *>(lds + slot * Geo::kStage + i * Geo::kStep +
+                                                           (o == 0 ? a0 : a1 + (o - 1) * 1024));
     };
-    uint32_t rdone = 0, rend = KB / NR;   // SEQ: ranges finished, end of the current one
-
-    auto step = [&](auto dc, uint32_t s) {   // K block s of the range, in ring slot d = s % kRing
-        constexpr uint32_t d = decltype(dc)::value;
-        // block s has landed and this wavefront has read all of block
-        // s-1 (whose slot the copies below take); then the same for all
-        __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(Geo::kPieces + kWLoads));
-        __builtin_amdgcn_s_barrier();
-        issue((d + 2) % kRing, s + 2);
-        __builtin_amdgcn_sched_barrier(0);
-        const uint8_t *const la = lds + d * Geo::kStage;
-        f32x16_t part[Geo::kOps];
+    auto cvt_b = [&](uint32_t slot, uint32_t i, uint32_t w) {   // dword w (0, 1) of step i's weights: two conversions
+        const uint32_t c = wbuf[slot][i / 2][2 * (i % 2) + w];
+        bop[i & 1][2 * w] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(c, 1.0f, false));
+        bop[i & 1][2 * w + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(c, 1.0f, true));
+    };
+    constexpr uint32_t kStageLoads = kPieces + Geo::kChunks;
+    __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((kRing - 1) * kStageLoads));
+    __builtin_amdgcn_s_barrier();
 #pragma unroll
-        for (uint32_t j = 0; j < 4; j++)
+    for (uint32_t o = 0; o < Geo::kOps; o++) read_a(0, 0, o);
+    cvt_b(0, 0, 0);
+    cvt_b(0, 0, 1);
+    auto step = [&](auto dc, uint32_t s) {   // stage s of the range, in ring slot d = s % kRing
+        constexpr uint32_t d = decltype(dc)::value, dn = (d + 1) % kRing;
+        constexpr uint32_t blk = d / Geo::kStages % 2;   // the K block's half of part
+        if constexpr (d % Geo::kStages == 0) {
+            sc_prev = sc_cur;
+            sc_cur = tab[s / Geo::kStages];
+        }
 #pragma unroll
-            for (uint32_t q = 0; q < 2; q++) {
-                const bf16x8_t bop = e4m3x8_to_bf16x8_cvt(wbuf[d][j][2 * q], wbuf[d][j][2 * q + 1], 1.0f);
-#pragma unroll
-                for (uint32_t o = 0; o < Geo::kOps; o++) {
-                    const uint32_t off = (j * 2 + q) * Geo::kStep + (o == 0 ? a0 : a1 + (o - 1) * 512);
-                    const bf16x8_t aop =
-                        __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const u32x4_t *>(la + off));
-                    part[o] = mfma32x32x16(aop, bop, j == 0 && q == 0 ? zero : part[o]);
-                }
+        for (uint32_t i = 0; i < kSteps; i++) {
+            if (i == kSteps - 1) {
+                // this wavefront has read all of stage s, whose slot the
+                // copies take, and stage s+1 has landed; then all have
+                __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((kRing - 2) * kStageLoads));
+                __builtin_amdgcn_s_barrier();
+                issue(d, s + kRing);
             }
-        const float scale = mytab[s];
+            __builtin_amdgcn_sched_barrier(0);
+            const uint32_t ns_slot = i == kSteps - 1 ? dn : d, ni = (i + 1) % kSteps;
 #pragma unroll
-        for (uint32_t o = 0; o < Geo::kOps; o++)
+            for (uint32_t o = 0; o < Geo::kOps; o++) {
+                part[blk][o] = mfma32x32x16(__builtin_bit_cast(bf16x8_t, aop[i & 1][o]),
+                                            __builtin_bit_cast(bf16x8_t, bop[i & 1]),
+                                            d % Geo::kStages == 0 && i == 0 ? zero : part[blk][o]);
+                read_a(ns_slot, ni, o);
+                if (o < 2) cvt_b(ns_slot, ni, o);
+                const uint32_t k = ((d % Geo::kStages) * kSteps + i) * Geo::kOps + o;
 #pragma unroll
-            for (uint32_t r = 0; r < (T == 16 && o == 1 ? 8u : 16u); r++)
-                acc[o][r] = __builtin_fmaf(scale, part[o][r], acc[o][r]);
-        if constexpr (SEQ) {
-            if (s + 1 == rend) {
-#pragma unroll
-                for (uint32_t r = 0; r < Geo::kRegs; r++) {
-                    const float v = range_sum(r);
-                    tot[r] = rdone ? tot[r] + v : v;
-                }
-#pragma unroll
-                for (uint32_t o = 0; o < Geo::kOps; o++) acc[o] = zero;
-                rdone++;
-                rend = (rdone + 1) * KB / NR;
+                for (uint32_t x = k * kSums / kSlots; x < (k + 1) * kSums / kSlots; x++)
+                    acc[x / 16][x % 16] = __builtin_fmaf(sc_prev, part[blk ^ 1][x / 16][x % 16], acc[x / 16][x % 16]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     };
@@ -277,79 +321,68 @@ void gemv_batch_kernel(BatchParams p) {
     // flight, also lead back to its start, and each turn would wait for the
     // newest weights.
     using std::integral_constant;
-    uint32_t b = 0;
-    for (; b + kRing <= n; b += kRing) {
-        step(integral_constant<uint32_t, 0>{}, b);
-        step(integral_constant<uint32_t, 1>{}, b + 1);
-        step(integral_constant<uint32_t, 2>{}, b + 2);
+    uint32_t s = 0;
+    for (; s + kRing <= ns; s += kRing) {
+        step(integral_constant<uint32_t, 0>{}, s);
+        step(integral_constant<uint32_t, 1>{}, s + 1);
+        step(integral_constant<uint32_t, 2>{}, s + 2);
+        step(integral_constant<uint32_t, 3>{}, s + 3);
     }
-    static_assert(kRing == 3, "steps of a turn");
-    if (b < n) step(integral_constant<uint32_t, 0>{}, b);
-    if (b + 1 < n) step(integral_constant<uint32_t, 1>{}, b + 1);
+    static_assert(kRing == 4, "steps of a turn");
+    if (s < ns) step(integral_constant<uint32_t, 0>{}, s);
+    if (s + 1 < ns) step(integral_constant<uint32_t, 1>{}, s + 1);
+    if constexpr (Geo::kStages == 1)
+        if (s + 2 < ns) step(integral_constant<uint32_t, 2>{}, s + 2);
     __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(0));   // no copy outlives the loop
+#pragma unroll
+    for (uint32_t x = 0; x < kSums; x++) {   // the last K block's sums
+        const float v = n & 1 ? part[0][x / 16][x % 16] : part[1][x / 16][x % 16];
+        acc[x / 16][x % 16] = __builtin_fmaf(sc_cur, v, acc[x / 16][x % 16]);
+    }
 
-    const uint32_t col = sub * kSubRows + mrow;      // weight row
-    auto token = [&](uint32_t r) { return tile * T + 8 * (r >> 2) + 4 * hh + (r & 3); };
-    if constexpr (!SEQ) {
-        float *dst = p.ws + sg.ws_off + (size_t)range * p.m * (sg.nb * kBlock) + col;
+    // per token row: (part 0 + part 1) + part 2
+    const size_t ld = (size_t)sg.nb * kBlock;
+    float *dst = p.ws + sg.ws_off + (size_t)range * p.m * ld + rg * kBlock + wv * kSubRows + mrow;
 #pragma unroll
-        for (uint32_t r = 0; r < Geo::kRegs; r++)
-            if (token(r) < p.m) dst[(size_t)token(r) * (sg.nb * kBlock)] = range_sum(r);
-    } else if constexpr (!PAIR) {
-#pragma unroll
-        for (uint32_t r = 0; r < Geo::kRegs; r++)
-            if (token(r) < p.m && col < sg.rows) {
-                const size_t o = (size_t)token(r) * sg.ldy + col;
-                sg.y[o] = sg.resid ? sg.resid[o] + tot[r] : tot[r];
-            }
-    } else {
-        // gate wavefront w and up wavefront w + 2 hold the same outputs:
-        // each hands half of its token rows to the other through LDS and
-        // forms silu(gate) * up of the other half
-        constexpr uint32_t H = Geo::kRegs / 2;
-        float *const xch = reinterpret_cast<float *>(lds);
-        const bool up = wv >= 2;
-        __builtin_amdgcn_s_barrier();   // every wavefront is done with the ring
-#pragma unroll
-        for (uint32_t r = 0; r < H; r++) xch[(wv * H + r) * 64 + lane] = up ? tot[r] : tot[r + H];
-        __syncthreads();
-#pragma unroll
-        for (uint32_t r = 0; r < H; r++) {
-            const float other = xch[((wv ^ 2) * H + r) * 64 + lane];
-            const float mine = up ? tot[r + H] : tot[r];
-            const uint32_t t = token(up ? r + H : r);
-            if (t < p.m && col < sg.rows)
-                p.seg[0].y[(size_t)t * sg.ldy + col] = swiglu1(up ? other : mine, up ? mine : other);
-        }
+    for (uint32_t r = 0; r < Geo::kRegs; r++) {
+        const uint32_t t = tile * T + 8 * (r >> 2) + 4 * hh + (r & 3);
+        const float v = T == 32 ? (acc[0][r] + acc[1][r]) + acc[Geo::kOps - 1][r]
+                                : (acc[0][r] + acc[0][(r + 8) & 15]) + acc[1][r];
+        if (t < p.m) dst[(size_t)t * ld] = v;
     }
 }
 
 // y = (resid +) the range sums of one segment, added in range order.
+template <uint32_t NR>
 __global__ __launch_bounds__(256) void batch_combine_kernel(BatchParams p) {
     const GemvSeg &sg = p.seg[blockIdx.z];
     const uint32_t row = blockIdx.x * 256 + threadIdx.x, t = blockIdx.y;
     if (row >= sg.rows) return;
-    const size_t ld = (size_t)sg.nb * kBlock;
+    const size_t ld = (size_t)sg.nb * kBlock, o = (size_t)t * sg.ldy + row;
     const float *src = p.ws + sg.ws_off + (size_t)t * ld + row;
-    float sum = src[0];
-    for (uint32_t r = 1; r < p.nr; r++) sum += src[(size_t)r * p.m * ld];
-    const size_t o = (size_t)t * sg.ldy + row;
-    sg.y[o] = sg.resid ? sg.resid[o] + sum : sum;
+    float v[NR];
+#pragma unroll
+    for (uint32_t r = 0; r < NR; r++) v[r] = src[(size_t)r * p.m * ld];
+    const float x = sg.resid ? sg.resid[o] : 0.0f;
+    float sum = v[0];
+#pragma unroll
+    for (uint32_t r = 1; r < NR; r++) sum += v[r];
+    sg.y[o] = sg.resid ? x + sum : sum;
 }
 
 uint32_t batch_tile(uint32_t m) { return m <= 16 ? 16 : 32; }
 
 size_t batch_act_bytes(uint32_t m, uint32_t kb) {
-    const uint32_t T = batch_tile(m);
-    const size_t blocks = (size_t)((m + T - 1) / T) * kb;
-    return blocks * (768 * T) + ((blocks * sizeof(float) + 255) & ~(size_t)255);
+    return (size_t)((m + 31) / 32) * kb * BatchGeo<32>::kBlk;
 }
 
-hipError_t launch_split_act(const float *x, uint32_t ldx, uint32_t m, uint32_t k, uint32_t kb, bool vec, uint8_t *xs,
-                            float *xf, hipStream_t stream) {
-    if (m == 0 || k == 0 || kb != (k + kBlock - 1) / kBlock || (vec && k % 8 != 0)) return hipErrorInvalidValue;
-    const uint32_t T = batch_tile(m);
-    const dim3 grid((m + T - 1) / T * kb), block(256);
+size_t batch_ws_floats(uint32_t m, uint32_t nb, uint32_t nr) { return (size_t)nr * m * nb * kBlock; }
+
+hipError_t launch_split_act(const float *x, uint32_t ldx, uint32_t m, uint32_t k, uint32_t kb, bool vec, uint32_t T,
+                            uint8_t *xs, float *xf, hipStream_t stream) {
+    if (m == 0 || k == 0 || kb != (k + kBlock - 1) / kBlock || (vec && k % 8 != 0) || (T != 16 && T != 32))
+        return hipErrorInvalidValue;
+    const dim3 grid((m + T - 1) / T * kb), block(16 * T);
     if (T == 16)
         hipLaunchKernelGGL((vec ? split_act_kernel<16, true> : split_act_kernel<16, false>), grid, block, 0, stream, x,
                            ldx, m, k, kb, xs, xf);
@@ -359,46 +392,46 @@ hipError_t launch_split_act(const float *x, uint32_t ldx, uint32_t m, uint32_t k
     return hipGetLastError();
 }
 
-hipError_t launch_gemv_batch(const BatchParams &pin, bool seq, bool pair, hipStream_t stream) {
+hipError_t launch_gemv_batch(const BatchParams &pin, bool combine, hipStream_t stream) {
     BatchParams p = pin;
-    if (p.m == 0 || p.nseg == 0 || p.nseg > 4 || !gemv_rows_shape(p.kb, p.nr) || (pair && (!seq || p.nseg != 2)))
+    const uint32_t T = p.tile;
+    if (p.m == 0 || p.nseg == 0 || p.nseg > 4 || (p.nr != 4 && p.nr != 8) ||
+        !gemv_rows_shape(p.kb, p.nr) || (T != 16 && T != 32))
         return hipErrorInvalidValue;
-    const uint32_t T = batch_tile(p.m);
     p.tiles = (p.m + T - 1) / T;
-    uint32_t groups = 0, max_rows = 0;
+    p.groups = 0;
+    uint32_t max_rows = 0;
     for (uint32_t s = 0; s < p.nseg; s++) {
-        p.seg[s].cta_begin = groups;
-        groups += p.seg[s].nb;
+        p.seg[s].cta_begin = p.groups;
+        p.groups += p.seg[s].nb;
         max_rows = std::max(max_rows, p.seg[s].rows);
     }
-    if (pair) {
-        if (p.seg[0].rows != p.seg[1].rows || p.seg[0].nb != p.seg[1].nb) return hipErrorInvalidValue;
-        groups = (p.seg[0].rows + 63) / 64;
-    }
-    p.groups = groups;
-    p.items = seq ? groups : groups * p.nr;
+    const dim3 grid((p.groups * p.nr + 7) / 8 * 8 * p.tiles);
+    const uint32_t lds = kRing * BatchGeo<16>::kStage + kGemvRsMaxKb * sizeof(float);
+    static_assert(BatchGeo<16>::kStage == BatchGeo<32>::kStage, "one ring size");
     using Kernel = void (*)(BatchParams);
-    static const Kernel kernels[6] = {gemv_batch_kernel<16, false, false>, gemv_batch_kernel<16, true, false>,
-                                      gemv_batch_kernel<16, true, true>,   gemv_batch_kernel<32, false, false>,
-                                      gemv_batch_kernel<32, true, false>,  gemv_batch_kernel<32, true, true>};
-    static bool attr_set = false;
-    if (!attr_set) {
-        for (Kernel k : kernels) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
-            if (e != hipSuccess) return e;
-        }
-        attr_set = true;
-    }
-    const uint32_t lds = kRing * 8 * 96 * T + (pair ? 2 : 1) * kGemvRsMaxKb * sizeof(float);
-    hipLaunchKernelGGL(kernels[(T == 32 ? 3 : 0) + (pair ? 2 : seq ? 1 : 0)], dim3((p.items + 7) / 8 * 8 * p.tiles),
-                       dim3(256), lds, stream, p);
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess && !seq) {
-        hipLaunchKernelGGL(batch_combine_kernel, dim3((max_rows + 255) / 256, p.m, p.nseg), dim3(256), 0, stream, p);
-        e = hipGetLastError();
-    }
-    return e;
+    static const Kernel kernels[4] = {gemv_batch_kernel<16, false>, gemv_batch_kernel<16, true>,
+                                      gemv_batch_kernel<32, false>, gemv_batch_kernel<32, true>};
+    hipLaunchKernelGGL(kernels[(T == 32 ? 2 : 0) + (p.tiles == 1 ? 1 : 0)], grid, dim3(256), lds, stream, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !combine) return e;
+    hipLaunchKernelGGL((p.nr == 4 ? batch_combine_kernel<4> : batch_combine_kernel<8>),
+                       dim3((max_rows + 255) / 256, p.m, p.nseg), dim3(256), 0, stream, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_batch_swiglu(const BatchParams &p, uint32_t kb, uint8_t *xs, float *xf, hipStream_t stream) {
+    const GemvSeg &g = p.seg[0], &u = p.seg[1];
+    if (p.m == 0 || p.nseg != 2 || g.rows != u.rows || g.nb != u.nb || kb != g.nb || (p.tile != 16 && p.tile != 32) ||
+        (p.nr != 4 && p.nr != 8))
+        return hipErrorInvalidValue;
+    const uint32_t T = p.tile;
+    const dim3 grid((p.m + T - 1) / T * kb);
+    using Kernel = void (*)(BatchParams, uint32_t, uint8_t *, float *);
+    const Kernel k = T == 16 ? (p.nr == 4 ? batch_swiglu_kernel<16, 4> : batch_swiglu_kernel<16, 8>)
+                             : (p.nr == 4 ? batch_swiglu_kernel<32, 4> : batch_swiglu_kernel<32, 8>);
+    hipLaunchKernelGGL(k, grid, dim3(16 * T), 0, stream, p, kb, xs, xf);
+    return hipGetLastError();
 }
 
 }  // namespace q35mm

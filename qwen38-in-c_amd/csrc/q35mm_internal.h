@@ -150,29 +150,35 @@ __host__ __device__ constexpr uint32_t pair_norm_stride(uint32_t k) { return (((
 hipError_t launch_gemv_pair(const GemvParams &p, bool norm, uint32_t cus, hipStream_t stream);
 
 // ---- batched decode (gemv_batch.hip), more than kGemvMaxM tokens -------
-// Row-split weights (gemv_rows_shape) at any m: the activations split once
-// into MFMA A operands, then 128-row groups x token tiles of 16 or 32, with
-// the bits of the row-split GEMV.  Segments: codes, scale, y, resid, rows,
-// ldy, nb (and ws_off when not seq); cta_begin is set by the launch.
+// Row-split weights (gemv_rows_shape) at any m, in passes of up to
+// kBatchTokens: the activations split once into MFMA A operands, then one
+// workgroup per 128-row group, K range and tile of 16 or 32 tokens, and a
+// kernel that adds the ranges; the bits of the row-split GEMV.  Segments:
+// codes, scale, y, resid, rows, ldy, nb, ws_off; cta_begin is set by the
+// launch.
+constexpr uint32_t kBatchTokens = 64;
 struct BatchParams {
     GemvSeg seg[4];
-    const uint8_t *xs;   // split activations (launch_split_act)
+    const uint8_t *xs;   // split activations
     const float *xf;     // scale factor per token tile and K block
-    float *ws;           // !seq: range sums, segment s at ws_off: [nr][m][nb*128]
+    float *ws;           // range sums, segment s at ws_off: [nr][m][nb*128]
     uint32_t m, kb, nseg;
     uint32_t nr;         // K ranges: the row-split GEMV's wavefronts (4 or 8)
-    uint32_t groups, items, tiles;   // set by the launch
+    uint32_t tile;       // tokens per tile (batch_tile), 16 or 32
+    uint32_t groups, tiles;   // set by the launch
 };
-// Split activations of m tokens x kb K blocks, then their scale factors.
-size_t batch_act_bytes(uint32_t m, uint32_t kb);
-uint32_t batch_tile(uint32_t m);   // tokens per tile
+uint32_t batch_tile(uint32_t m);                                 // tokens per tile
+size_t batch_act_bytes(uint32_t m, uint32_t kb);                 // split activations, either tile
+size_t batch_ws_floats(uint32_t m, uint32_t nb, uint32_t nr);    // range sums of one segment
 // vec: rows of x 16-byte aligned and k % 8 == 0.
-hipError_t launch_split_act(const float *x, uint32_t ldx, uint32_t m, uint32_t k, uint32_t kb, bool vec, uint8_t *xs,
-                            float *xf, hipStream_t stream);
-// seq: a workgroup runs all K ranges of its rows; otherwise one workgroup
-// per range and a kernel that adds the range sums.  pair (seq): segments
-// gate and up of one shape, writing silu(gate) * up to seg[0].y.
-hipError_t launch_gemv_batch(const BatchParams &p, bool seq, bool pair, hipStream_t stream);
+hipError_t launch_split_act(const float *x, uint32_t ldx, uint32_t m, uint32_t k, uint32_t kb, bool vec,
+                            uint32_t tile, uint8_t *xs, float *xf, hipStream_t stream);
+// combine: also add the ranges into y; otherwise the range sums stay in ws
+// for launch_batch_swiglu.
+hipError_t launch_gemv_batch(const BatchParams &p, bool combine, hipStream_t stream);
+// silu(segment 0) * segment 1 of the range sums, split into the activations
+// of a weight of kb K blocks (kb*128 >= rows).
+hipError_t launch_batch_swiglu(const BatchParams &p, uint32_t kb, uint8_t *xs, float *xf, hipStream_t stream);
 
 // ---- chained decode GEMVs (chain.hip) ---------------------------------
 // One step: a row-split GEMV over 1..4 weights sharing x.  seg[i].cta_begin

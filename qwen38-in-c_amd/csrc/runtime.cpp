@@ -519,64 +519,78 @@ int run_gemv_group(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
     return Q35MM_OK;
 }
 
-// Batched decode of row-split weights (gemv_batch.hip): m > kGemvMaxM tokens
-// in passes of up to kBatchTokens (bounds the workspace).  pair: w is gate
-// and up of one shape and dY[0] receives silu(gate) * up.  Returns kNoRoom,
-// with nothing launched, when there is no scratch for it -- a capture on a
-// stream without a set of its own (scr null) or with too small a one, or the
-// fixed scratch of an allocation-free call -- and the caller takes the
-// launches of eight tokens, which need none and give the same bits.
-constexpr uint32_t kBatchTokens = 64;
+// Batched decode (gemv_batch.hip) of row-split weights: scratch for passes
+// of mp tokens over weights of up to kb K blocks and nb row groups in all.
+// xs and xf share the GEMM's activation buffer.  kNoRoom, with nothing
+// launched, when there is no scratch for it -- a capture on a stream without
+// a set of its own (own false) or with too small a one, or the fixed scratch
+// of an allocation-free call -- and the caller takes the launches of eight
+// tokens, which need none and give the same bits.
 constexpr int kNoRoom = -1001;   // internal
 
+int batch_scratch(Scratch &sc, bool own, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t **xs, float **xf, float **ws) {
+    if (!own && sc.capturing) return kNoRoom;
+    const size_t ab = batch_act_bytes(mp, kb), fb = 2 * (size_t)kb * sizeof(float);   // at most two tiles
+    const size_t xb = (ab + fb + 255) & ~(size_t)255, wb = batch_ws_floats(mp, nb, g_dev.rows_waves) * sizeof(float);
+    if (sc.fixed ? xb + wb > kNoAllocBytes : sc.capturing && (sc.xb.cap < xb || sc.ws.cap < wb)) return kNoRoom;
+    uint16_t *x = nullptr;
+    const int rc = scratch_gemm(sc, xb, wb, &x, ws);
+    if (rc) return rc;
+    *xs = reinterpret_cast<uint8_t *>(x);
+    *xf = reinterpret_cast<float *>(*xs + ab);
+    return Q35MM_OK;
+}
+
+// One weight of a batched pass of p.m tokens; returns the next one's ws_off.
+uint32_t batch_seg(BatchParams &p, uint32_t s, const Weight &w, float *y, const float *resid, uint32_t ws_off) {
+    GemvSeg &g = p.seg[s];
+    g = GemvSeg{};
+    g.codes = w.codes;
+    g.scale = w.scale;
+    g.y = y;
+    g.resid = resid;
+    g.rows = w.rows;
+    g.ldy = w.rows;
+    g.nb = w.nb;
+    g.ws_off = ws_off;
+    return ws_off + (uint32_t)batch_ws_floats(p.m, w.nb, p.nr);
+}
+
 int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const float *dX, float *const *dY,
-                   hipStream_t st, float *const *resid, Scratch *scr, bool pair) {
+                   hipStream_t st, float *const *resid, Scratch *scr) {
     Scratch &sc = scr ? *scr : scratch_for(st);
-    if (!scr && sc.capturing && !g_dev.scratch.count(st)) return kNoRoom;
-    const uint32_t cols = w[0]->w.cols, kb = w[0]->w.kb, mp = std::min(m, kBatchTokens);
-    uint32_t groups = 0, wsoff = 0;
+    const uint32_t cols = w[0]->w.cols, kb = w[0]->w.kb;
+    uint64_t nb = 0;
+    for (uint32_t s = 0; s < nseg; s++) nb += w[s]->w.nb;
     BatchParams p{};
     p.kb = kb;
     p.nseg = nseg;
     p.nr = g_dev.rows_waves;
-    for (uint32_t s = 0; s < nseg; s++) groups += w[s]->w.nb;
-    // A workgroup per row group and token tile where that gives every CU one;
-    // otherwise one per K range too, their sums added by a second kernel.
-    bool seq = pair || groups * ((mp + batch_tile(mp) - 1) / batch_tile(mp)) >= g_dev.cus;
-    for (uint32_t s = 0; s < nseg; s++) {
-        const Weight &ws = w[s]->w;
-        GemvSeg &g = p.seg[s];
-        g.codes = ws.codes;
-        g.scale = ws.scale;
-        g.rows = ws.rows;
-        g.ldy = ws.rows;
-        g.nb = ws.nb;
-        g.ws_off = wsoff;
-        wsoff += p.nr * mp * ws.nb * kBlock;
+    // tokens per pass: fewer where the range sums pass ws_off's 32 bits or
+    // the fixed scratch of an allocation-free call
+    uint32_t mp = std::min(m, kBatchTokens);
+    uint8_t *xs = nullptr;
+    float *xf = nullptr;
+    int rc = kNoRoom;
+    for (; rc == kNoRoom && mp > kGemvMaxM; mp = mp > 32 ? 32 : mp > 16 ? 16 : 0) {
+        if (batch_ws_floats(mp, 1, p.nr) * nb > UINT32_MAX) continue;
+        rc = batch_scratch(sc, scr || g_dev.scratch.count(st), mp, kb, (uint32_t)nb, &xs, &xf, &p.ws);
+        if (rc != kNoRoom) break;
     }
-    const size_t xb = (batch_act_bytes(mp, kb) + 255) & ~(size_t)255;
-    size_t wsb = (size_t)wsoff * sizeof(float);
-    if (sc.fixed && xb + wsb > kNoAllocBytes) seq = true;
-    if (seq) wsb = 0;
-    if (sc.fixed ? xb + wsb > kNoAllocBytes : sc.capturing && (sc.xb.cap < xb || sc.ws.cap < wsb)) return kNoRoom;
-    uint16_t *xs = nullptr;
-    const int rc = scratch_gemm(sc, xb, wsb, &xs, &p.ws);
     if (rc) return rc;
-    p.xs = reinterpret_cast<const uint8_t *>(xs);
+    p.xs = xs;
+    p.xf = xf;
     const bool vec = aligned16(dX) && cols % 8 == 0;
     for (uint32_t t0 = 0; t0 < m; t0 += mp) {
         p.m = std::min(mp, m - t0);
-        const uint32_t T = batch_tile(p.m);
-        float *xf = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(xs) +
-                                              (size_t)((p.m + T - 1) / T) * kb * 768 * T);
-        p.xf = xf;
+        uint32_t off = 0;
         for (uint32_t s = 0; s < nseg; s++) {
-            const size_t o = (size_t)t0 * p.seg[s].ldy;
-            p.seg[s].y = dY[pair ? 0 : s] + o;
-            p.seg[s].resid = resid ? resid[s] + o : nullptr;
+            const size_t o = (size_t)t0 * w[s]->w.rows;
+            off = batch_seg(p, s, w[s]->w, dY[s] + o, resid ? resid[s] + o : nullptr, off);
         }
-        HIP_TRY(launch_split_act(dX + (size_t)t0 * cols, cols, p.m, cols, kb, vec, reinterpret_cast<uint8_t *>(xs), xf, st));
-        HIP_TRY(launch_gemv_batch(p, seq, pair, st));
+        p.tile = batch_tile(p.m);
+        HIP_TRY(launch_split_act(dX + (size_t)t0 * cols, cols, p.m, cols, kb, vec, p.tile, xs, xf, st));
+        HIP_TRY(launch_gemv_batch(p, true, st));
     }
     return Q35MM_OK;
 }
@@ -589,7 +603,7 @@ int run_gemv(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const floa
              float *const *resid = nullptr, Scratch *scr = nullptr) {
     const uint32_t cols = w[0]->w.cols;
     if (m > kGemvMaxM && in.xmode == kXPlain && uses_gemv_rows(w[0]->w)) {   // same K: one kind for all
-        const int rc = run_gemv_batch(w, nseg, m, dX, dY, st, resid, scr, false);
+        const int rc = run_gemv_batch(w, nseg, m, dX, dY, st, resid, scr);
         if (rc != kNoRoom) return rc;
     }
     for (uint32_t t0 = 0; t0 < m; t0 += kGemvMaxM) {
@@ -1760,6 +1774,41 @@ int run_mlp_pair(const q35mm_weight *gate, const q35mm_weight *up, uint32_t m, c
     return Q35MM_OK;
 }
 
+// x += down(silu(xn @ gate^T) * (xn @ up^T)) for more than kGemvMaxM tokens
+// of row-split weights: the gate and up products' range sums become the down
+// product's split activations in one kernel.  Bits as above; kNoRoom as
+// batch_scratch.
+int run_mlp_batch(const q35mm_weight *gate, const q35mm_weight *up, const q35mm_weight *down, uint32_t m,
+                  const float *xn, float *dX, hipStream_t st, Scratch &scr) {
+    const Weight &g = gate->w, &u = up->w, &d = down->w;
+    const uint32_t H = g.cols, mp = std::min(m, kBatchTokens), kb = std::max(g.kb, d.kb), nb = std::max(2 * g.nb, d.nb);
+    BatchParams p{};
+    p.nr = g_dev.rows_waves;
+    if (batch_ws_floats(mp, nb, p.nr) > UINT32_MAX) return kNoRoom;
+    uint8_t *xs = nullptr;
+    float *xf = nullptr;
+    const int rc = batch_scratch(scr, true, mp, kb, nb, &xs, &xf, &p.ws);
+    if (rc) return rc;
+    p.xs = xs;
+    p.xf = xf;
+    for (uint32_t t0 = 0; t0 < m; t0 += mp) {
+        float *const x = dX + (size_t)t0 * H;
+        p.m = std::min(mp, m - t0);
+        p.kb = g.kb;
+        p.nseg = 2;
+        batch_seg(p, 1, u, nullptr, nullptr, batch_seg(p, 0, g, nullptr, nullptr, 0));
+        p.tile = batch_tile(p.m);
+        HIP_TRY(launch_split_act(xn + (size_t)t0 * H, H, p.m, H, g.kb, aligned16(xn) && H % 8 == 0, p.tile, xs, xf, st));
+        HIP_TRY(launch_gemv_batch(p, false, st));
+        HIP_TRY(launch_batch_swiglu(p, d.kb, xs, xf, st));
+        p.kb = d.kb;
+        p.nseg = 1;
+        batch_seg(p, 0, d, x, x, 0);
+        HIP_TRY(launch_gemv_batch(p, true, st));
+    }
+    return Q35MM_OK;
+}
+
 Q35MM_API int q35mm_mlp(const q35mm_weight *gate, const q35mm_weight *up, const q35mm_weight *down,
                         const float *dNormW, float eps, uint32_t m, float *dX, void *stream) {
     std::lock_guard<std::recursive_mutex> lk(g_mu);
@@ -1805,14 +1854,15 @@ Q35MM_API int q35mm_mlp(const q35mm_weight *gate, const q35mm_weight *up, const 
             // residual add.
             const bool norm_in = m == 1 && H <= kPairNormMaxCols && g_dev.mlp_pair == 1;
             if (!norm_in) HIP_TRY(launch_rmsnorm(dX, H, dNormW, xn, H, m, H, eps, st));
-            const q35mm_weight *gu[2] = {gate, up};
-            rc = m > kGemvMaxM ? run_gemv_batch(gu, 2, m, xn, &g, st, nullptr, &scr, true) : kNoRoom;
-            if (rc && rc != kNoRoom) return rc;
-            for (uint32_t t0 = 0; rc == kNoRoom && t0 < m; t0 += kGemvMaxM) {
+            if (m > kGemvMaxM && uses_gemv_rows(down->w)) {
+                rc = run_mlp_batch(gate, up, down, m, xn, dX, st, scr);
+                if (rc != kNoRoom) return rc;
+            }
+            for (uint32_t t0 = 0; t0 < m; t0 += kGemvMaxM) {
                 const uint32_t mt = std::min(kGemvMaxM, m - t0);
-                const int e = run_mlp_pair(gate, up, mt, (norm_in ? dX : xn) + (size_t)t0 * H,
-                                           norm_in ? dNormW : nullptr, eps, g + (size_t)t0 * I, st);
-                if (e) return e;
+                rc = run_mlp_pair(gate, up, mt, (norm_in ? dX : xn) + (size_t)t0 * H, norm_in ? dNormW : nullptr, eps,
+                                  g + (size_t)t0 * I, st);
+                if (rc) return rc;
             }
             return run_gemv(dn, 1, m, g, dy, st, GemvInput(), dy, &scr);
         }
