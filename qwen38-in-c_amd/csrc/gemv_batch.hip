@@ -11,24 +11,37 @@
 // splits the activations of its K range again.  Here
 //  - split_act_kernel splits the activations once, exactly, into three bf16
 //    parts and writes them in MFMA A-operand order;
-//  - a workgroup owns a 128-row group of one weight (four wavefronts, one
-//    32-row sub-tile each) for a tile of T = 16 or 32 tokens.  It streams the
-//    weights HBM -> registers two K blocks ahead and copies each K block's
-//    split activations (12 or 24 KiB, shared by the four wavefronts) into a
-//    three-deep LDS ring with global_load_lds.  Matrix work per weight byte
-//    is what bounds it then: 24 MFMAs per 4 KiB sub-tile at T = 32 are 768
-//    cycles of a SIMD's matrix core, which for a layer's 383 MB is 29 us at
-//    32 tokens against 76 us of HBM traffic at 5 TB/s;
+//  - a workgroup owns one K range (the NR = 4 or 8 ranges the row-split
+//    GEMV's wavefronts have) of a 128-row group, four wavefronts with one
+//    32-row sub-tile each, for a tile of T = 16 or 32 tokens.  It streams the
+//    weights HBM -> registers and the split activations, shared by the four
+//    wavefronts, into an LDS ring, both four stages ahead;
 //  - tokens beyond one tile are further workgroups of the same launch, placed
-//    so that the workgroups of one row group share an XCD's L2.
+//    so that those of one row group share an XCD's L2 (plain weight loads
+//    then: 61 tokens of 5120 -> 14336 32.8 us against 38.9 non-temporal);
+//  - the range sums (fp32) go to memory and batch_combine_kernel adds them in
+//    range order, or, of an MLP's gate and up, batch_swiglu_kernel adds them
+//    and writes silu(gate) * up already split for the down product.
 //
-// Bits.  The decode GEMV sums each of its NR (4 or 8) K ranges block by block
-// (one fmaf with the block's scale per block and part), adds the three parts,
-// then the ranges in order.  Every step is kept: MFMA A rows only select
-// tokens and parts, so which rows they sit in does not change a sum.
-// Ranges either run one after another in one workgroup (SEQ) or as NR
-// workgroups whose sums batch_combine_kernel adds in range order; the bits
-// are the same.
+// What bounds it: at 24 tokens (T = 32) gate and up of 5120 -> 2 x 17408
+// (178 MB) take 50 us, 3.5 TB/s; HBM alone would take 30.  The CU's pipes are
+// all busy half the time or more and overlap in part: per K block a SIMD's
+// wavefront has 24 MFMAs (768 cycles), ~450 cycles of conversions and
+// scaling, 24 LDS reads, and the CU copies 24 KiB of activations beside its
+// 16 KiB of weights.  Ranges one after another in one workgroup instead (272
+// workgroups for the same launch, no range sums) took 65.8 us: two chains on
+// some CUs, one on the others.  Down (17408 -> 5120, 160 workgroups, 26 us)
+// is bound by each wavefront's chain of 34 K blocks.
+//
+// Whole calls against the row-split GEMV in groups of eight, us: 5120 ->
+// 16480 at 24 tokens 66.8 -> 36.8, at 63 tokens 178.8 -> 51.5; 17408 -> 5120
+// 77.5 -> 37.5 and 207.8 -> 56.0.  (The runtime's batch_pays says from which
+// sizes on it is taken.)
+//
+// Bits.  The decode GEMV sums each of its K ranges block by block (one fmaf
+// with the block's scale per block and part), adds the three parts, then the
+// ranges in order.  Every step is kept: MFMA A rows only select tokens and
+// parts, so which rows they sit in does not change a sum.
 #include <algorithm>
 #include <type_traits>
 

@@ -528,6 +528,19 @@ int run_gemv_group(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
 // tokens, which need none and give the same bits.
 constexpr int kNoRoom = -1001;   // internal
 
+// Whether m tokens of row-split weights go as one batch.  From 17 tokens on
+// always: the three launches of a batch replace three or more of the
+// eight-token GEMV (1024 x 1024: 13.5 us either way at 17 tokens, 33.0 ->
+// 13.5 at 63).  9..16 tokens are two such launches, which a batch beats only
+// if each runs long enough: 9 tokens of 3072 -> 1024 11.9 us as two launches,
+// 13.1 as a batch, 4096 -> 1024 14.2 and 12.9, 5120 -> 16480 41.8 and 30.3.
+// kb: the weight's K blocks; of an MLP block (which runs one launch more
+// than its eight-token form, not counting repeats) gate's plus down's: 9
+// tokens of 512 -> 1664 21.0 and 23.2 us, 2048 -> 2048 25.7 and 25.8, 4096
+// -> 4096 36.0 and 34.6, 5120 -> 17408 119.7 and 86.9.
+constexpr uint32_t kBatchMinKb = 28, kBatchMinKbMlp = 33;
+bool batch_pays(uint32_t m, uint32_t kb, uint32_t min_kb) { return m > 2 * kGemvMaxM || (m > kGemvMaxM && kb >= min_kb); }
+
 int batch_scratch(Scratch &sc, bool own, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t **xs, float **xf, float **ws) {
     if (!own && sc.capturing) return kNoRoom;
     const size_t ab = batch_act_bytes(mp, kb), fb = 2 * (size_t)kb * sizeof(float);   // at most two tiles
@@ -595,14 +608,14 @@ int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
     return Q35MM_OK;
 }
 
-// Weights sharing K: more than eight tokens of row-split weights as one
-// batch, everything else in groups of up to eight tokens; stream-K weights
+// Weights sharing K: row-split weights as one batch where that pays,
+// everything else in groups of up to eight tokens; stream-K weights
 // share one launch, row-split weights another.
 int run_gemv(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const float *dX,
              float *const *dY, hipStream_t st, const GemvInput &in = GemvInput(),
              float *const *resid = nullptr, Scratch *scr = nullptr) {
     const uint32_t cols = w[0]->w.cols;
-    if (m > kGemvMaxM && in.xmode == kXPlain && uses_gemv_rows(w[0]->w)) {   // same K: one kind for all
+    if (batch_pays(m, w[0]->w.kb, kBatchMinKb) && in.xmode == kXPlain && uses_gemv_rows(w[0]->w)) {   // same K: one kind
         const int rc = run_gemv_batch(w, nseg, m, dX, dY, st, resid, scr);
         if (rc != kNoRoom) return rc;
     }
@@ -1854,7 +1867,7 @@ Q35MM_API int q35mm_mlp(const q35mm_weight *gate, const q35mm_weight *up, const 
             // residual add.
             const bool norm_in = m == 1 && H <= kPairNormMaxCols && g_dev.mlp_pair == 1;
             if (!norm_in) HIP_TRY(launch_rmsnorm(dX, H, dNormW, xn, H, m, H, eps, st));
-            if (m > kGemvMaxM && uses_gemv_rows(down->w)) {
+            if (batch_pays(m, gate->w.kb + down->w.kb, kBatchMinKbMlp) && uses_gemv_rows(down->w)) {
                 rc = run_mlp_batch(gate, up, down, m, xn, dX, st, scr);
                 if (rc != kNoRoom) return rc;
             }

@@ -30,9 +30,11 @@ def _same_bits(a, b):
     assert torch.equal(a.view(torch.int32), b.view(torch.int32))
 
 
-@pytest.mark.parametrize("m,k,rows", [(9, 400, (200,)), (16, 1003, (4100,)), (17, 5120, (1024,)), (32, 640, (33000,)),
+# 9..16 tokens: 28 K blocks or more (fewer go as two small calls)
+@pytest.mark.parametrize("m,k,rows", [(9, 3600, (200,)), (16, 4571, (4100,)), (12, 5120, (1300, 48, 5000)),
+                                      (10, 20480, (1,)), (17, 5120, (1024,)), (32, 640, (33000,)), (18, 400, (70,)),
                                       (33, 20480, (129,)), (63, 17400, (300,)), (24, 1032, (130, 48, 1, 5000)),
-                                      (12, 897, (20000, 16000)), (63, 768, (16300, 70)), (10, 512, (1,))])
+                                      (63, 768, (16300, 70)), (16, 3456, (300,)), (9, 3457, (300,))])
 def test_batch_rows_are_small_calls_bitwise(q, wl, gpu, m, k, rows):
     import torch
     ws = [q.Weight(*wl.gen_weight_ragged(k + i, n, k)) for i, n in enumerate(rows)]
@@ -57,7 +59,7 @@ def test_batch_rows_are_small_calls_bitwise(q, wl, gpu, m, k, rows):
 def test_batch_wide_values(q, wl, gpu, m):
     """Blocks holding values past 2^96 or infinities are staged shifted."""
     import torch
-    k, n = 1000, 300
+    k, n = 3600, 300
     w = q.Weight(*wl.gen_weight(5, n, k))
     X = wl.gen_act(6, m, k)
     X[0, 3], X[1, 700], X[2, 999] = np.inf, -np.inf, np.float32(3.4e38)
@@ -71,7 +73,7 @@ def test_batch_wide_values(q, wl, gpu, m):
     w.free()
 
 
-@pytest.mark.parametrize("m,H,I", [(9, 640, 1664), (16, 1032, 4100), (31, 5120, 1000), (63, 512, 16400)])
+@pytest.mark.parametrize("m,H,I", [(9, 3600, 1664), (16, 1032, 4100), (12, 640, 1664), (31, 5120, 1000), (63, 512, 16400)])
 def test_batch_mlp_is_small_calls_bitwise(q, wl, gpu, m, H, I):
     """Gate and up in one pass forming silu(gate) * up; residual added."""
     import torch
