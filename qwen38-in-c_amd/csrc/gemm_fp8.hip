@@ -298,6 +298,22 @@ __device__ __forceinline__ void store_act_bf16(uint16_t *act, uint32_t act_kb, u
         (uint16_t)(f32x2_to_bf16x2_rne(v, 0.0f) & 0xFFFFu);
 }
 
+// Activations of tokens t (v0) and t + 1 (v1) at column c, t even, where
+// lane ^ 1 holds the same tokens of column c ^ 1: the pair of lanes trades
+// halves, so the even lane stores both columns of token t and the odd lane
+// both of t + 1 -- one 4-byte store a lane in place of two of 2 bytes.
+__device__ __forceinline__ void store_act_bf16_pair(uint16_t *act, uint32_t act_kb, uint32_t t, uint32_t c, float v0,
+                                                    float v1) {
+    const uint32_t own = f32x2_to_bf16x2_rne(v0, v1);
+    const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)own, 0xB1, 0xF, 0xF, true);   // quad_perm 1,0,3,2
+    const bool odd = c & 1;
+    const uint32_t pair = odd ? (other >> 16) | (own & 0xFFFF0000u) : (own & 0xFFFFu) | (other << 16);
+    const uint32_t tt = t + (odd ? 1 : 0), cc = (c % kBlock) & ~1u;
+    const uint32_t u = ((cc >> 5) * 2 + ((cc >> 3) & 1)) * 64 + ((cc >> 4) & 1) * 32 + tt % 32;
+    *reinterpret_cast<uint32_t *>(act + ((size_t)(tt / 32) * act_kb + c / kBlock) * (4 * kChunkBytes) + u * 8 + (cc & 7)) =
+        pair;
+}
+
 // silu(g) * u of a paired tile, as act_to_bf16_kernel<true> forms it before
 // rounding.
 __device__ __forceinline__ float paired_swiglu(float g, float u) { return bf16_saturate(swiglu1(g, u)); }
@@ -851,15 +867,19 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_fp8_kernel(GemmParams p) {
 #pragma unroll
                         for (uint32_t jn = 0; jn < kTN; jn++)
 #pragma unroll
-                            for (uint32_t e = 0; e < 16; e++) {
-                                const float own = acc[base + ii][jn][e], other = xat(1 - hs, ii * 2 + jn, e);
+                            for (uint32_t e = 0; e < 16; e += 2) {
                                 const uint32_t mrow = mt * Geo::kTM + out_row(base + ii, e);
                                 const uint32_t ncol = pcol(jn);
-                                if (ncol < p.act_kb * kBlock)
-                                    store_act_bf16(p.act_out, p.act_kb, mrow, ncol,
-                                                   mrow < p.m && ncol < sg.rows
-                                                       ? paired_swiglu(hs ? other : own, hs ? own : other)
-                                                       : 0.0f);
+                                float y[2];
+#pragma unroll
+                                for (uint32_t z = 0; z < 2; z++) {
+                                    const float own = acc[base + ii][jn][e + z], other = xat(1 - hs, ii * 2 + jn, e + z);
+                                    y[z] = mrow + z < p.m && ncol < sg.rows
+                                               ? paired_swiglu(hs ? other : own, hs ? own : other)
+                                               : 0.0f;
+                                }
+                                if (ncol < p.act_kb * kBlock)   // the same for both columns of a pair
+                                    store_act_bf16_pair(p.act_out, p.act_kb, mrow, ncol, y[0], y[1]);
                             }
                 };
                 __syncthreads();   // every wavefront is done reading the ring
