@@ -522,10 +522,9 @@ int run_gemv_group(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
 // Batched decode (gemv_batch.hip) of row-split weights: scratch for passes
 // of mp tokens over weights of up to kb K blocks and nb row groups in all.
 // xs and xf share the GEMM's activation buffer.  kNoRoom, with nothing
-// launched, when there is no scratch for it -- a capture on a stream without
-// a set of its own (own false) or with too small a one, or the fixed scratch
-// of an allocation-free call -- and the caller takes the launches of eight
-// tokens, which need none and give the same bits.
+// launched, when there is no scratch for it (the fixed scratch of an
+// allocation-free call), and the caller takes the launches of eight tokens,
+// which need none and give the same bits.
 constexpr int kNoRoom = -1001;   // internal
 
 // Whether m tokens of row-split weights go as one batch.  From 17 tokens on
@@ -541,11 +540,22 @@ constexpr int kNoRoom = -1001;   // internal
 constexpr uint32_t kBatchMinKb = 28, kBatchMinKbMlp = 33;
 bool batch_pays(uint32_t m, uint32_t kb, uint32_t min_kb) { return m > 2 * kGemvMaxM || (m > kGemvMaxM && kb >= min_kb); }
 
-int batch_scratch(Scratch &sc, bool own, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t **xs, float **xf, float **ws) {
-    if (!own && sc.capturing) return kNoRoom;
+// Whether calls on st may use the batch's scratch.  Not in a graph capture:
+// a graph may be replayed on any stream, beside eager calls on the captured
+// one and other graphs, which would overwrite that scratch; the launches of
+// eight tokens hold none.  A stream that cannot be asked (the null stream
+// while another is captured) counts as captured.
+bool batch_allowed(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();   // or the next launch would report it
+    return false;
+}
+
+int batch_scratch(Scratch &sc, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t **xs, float **xf, float **ws) {
     const size_t ab = batch_act_bytes(mp, kb), fb = 2 * (size_t)kb * sizeof(float);   // at most two tiles
     const size_t xb = (ab + fb + 255) & ~(size_t)255, wb = batch_ws_floats(mp, nb, g_dev.rows_waves) * sizeof(float);
-    if (sc.fixed ? xb + wb > kNoAllocBytes : sc.capturing && (sc.xb.cap < xb || sc.ws.cap < wb)) return kNoRoom;
+    if (sc.fixed && xb + wb > kNoAllocBytes) return kNoRoom;
     uint16_t *x = nullptr;
     const int rc = scratch_gemm(sc, xb, wb, &x, ws);
     if (rc) return rc;
@@ -571,6 +581,7 @@ uint32_t batch_seg(BatchParams &p, uint32_t s, const Weight &w, float *y, const 
 
 int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const float *dX, float *const *dY,
                    hipStream_t st, float *const *resid, Scratch *scr) {
+    if (!batch_allowed(st)) return kNoRoom;
     Scratch &sc = scr ? *scr : scratch_for(st);
     const uint32_t cols = w[0]->w.cols, kb = w[0]->w.kb;
     uint64_t nb = 0;
@@ -587,7 +598,7 @@ int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
     int rc = kNoRoom;
     for (; rc == kNoRoom && mp > kGemvMaxM; mp = mp > 32 ? 32 : mp > 16 ? 16 : 0) {
         if (batch_ws_floats(mp, 1, p.nr) * nb > UINT32_MAX) continue;
-        rc = batch_scratch(sc, scr || g_dev.scratch.count(st), mp, kb, (uint32_t)nb, &xs, &xf, &p.ws);
+        rc = batch_scratch(sc, mp, kb, (uint32_t)nb, &xs, &xf, &p.ws);
         if (rc != kNoRoom) break;
     }
     if (rc) return rc;
@@ -1797,10 +1808,10 @@ int run_mlp_batch(const q35mm_weight *gate, const q35mm_weight *up, const q35mm_
     const uint32_t H = g.cols, mp = std::min(m, kBatchTokens), kb = std::max(g.kb, d.kb), nb = std::max(2 * g.nb, d.nb);
     BatchParams p{};
     p.nr = g_dev.rows_waves;
-    if (batch_ws_floats(mp, nb, p.nr) > UINT32_MAX) return kNoRoom;
+    if (!batch_allowed(st) || batch_ws_floats(mp, nb, p.nr) > UINT32_MAX) return kNoRoom;
     uint8_t *xs = nullptr;
     float *xf = nullptr;
-    const int rc = batch_scratch(scr, true, mp, kb, nb, &xs, &xf, &p.ws);
+    const int rc = batch_scratch(scr, mp, kb, nb, &xs, &xf, &p.ws);
     if (rc) return rc;
     p.xs = xs;
     p.xf = xf;

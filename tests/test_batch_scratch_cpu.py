@@ -1,0 +1,127 @@
+"""Scratch of the batched decode (9..63 tokens of row-split weights) in the
+host code: runtime.cpp linked to a recording stand-in for HIP and the kernel
+launches (tests/c/host_stub.cpp), so every launch's scratch pointers, and
+every allocation, free and wait of a call are seen without a GPU.
+
+One to eight tokens of a row-split weight need no scratch, and neither did
+batches launched eight tokens at a time: a HIP graph of them can be replayed
+on any stream beside any other work.  The batch keeps that by never being
+captured.
+"""
+import ctypes as C
+import os
+import shutil
+import subprocess
+
+import numpy as np
+import pytest
+
+from conftest import ROOT
+
+CSRC = os.path.join(ROOT, "qwen38-in-c_amd", "csrc")
+S, T, U = 0x1000, 0x2000, 0x3000   # streams
+
+
+@pytest.fixture(scope="module")
+def stub_path(tmp_path_factory):
+    if not shutil.which("g++") or not os.path.exists("/opt/rocm/include/hip/hip_runtime.h"):
+        pytest.skip("g++ and the HIP headers needed")
+    so = str(tmp_path_factory.mktemp("stub") / "libhoststub.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I", os.path.join(ROOT, "include"), "-I", CSRC, "-fPIC", "-shared", "-fvisibility=hidden",
+                    "-Wl,-Bsymbolic", "-Wl,--no-undefined", "-o", so, os.path.join(ROOT, "tests", "c", "host_stub.cpp"),
+                    os.path.join(CSRC, "runtime.cpp"), os.path.join(CSRC, "safetensors.cpp"), "-lpthread", "-ldl"],
+                   check=True)
+    return so
+
+
+class Lib:
+    """The library over the stand-in; addresses in place of device tensors."""
+
+    def __init__(self, path):
+        import q35mm
+        self.lib = q35mm._load(path)
+        self.lib.stub_log.restype = C.c_char_p
+        self.lib.stub_capture.argtypes = [C.c_void_p, C.c_int]
+        self.lib.stub_fail_malloc.argtypes = [C.c_size_t]
+        self.x, self.y = 1 << 40, 1 << 41
+        assert self.lib.q35mm_init(0) == 0
+        self.take()
+
+    def weight(self, rows, cols, wide=False):
+        W = np.zeros((rows, cols), np.uint8)
+        sc = np.full(((rows + 127) // 128, (cols + 127) // 128), 0x3F80, np.uint16)
+        if wide:
+            sc[0, 0], sc[0, 1] = 0x6F80, 0x3380     # 2^96 and 2^-24: beyond the GEMM
+        w = C.c_void_p()
+        p8, p16 = C.POINTER(C.c_uint8), C.POINTER(C.c_uint16)
+        assert self.lib.q35mm_weight_create(W.ctypes.data_as(p8), sc.ctypes.data_as(p16), rows, cols, C.byref(w)) == 0
+        self.take()
+        return w
+
+    def take(self):
+        """The recorded lines since the last take: (kind, {key: value})."""
+        lines = self.lib.stub_log().decode().splitlines()
+        self.lib.stub_clear()
+        return [(ln.split()[0], dict(f.split("=") for f in ln.split() if "=" in f), ln) for ln in lines]
+
+    def matmul(self, w, m, st):
+        return self.lib.q35mm_matmul(w, m, self.x, self.y, st), self.take()
+
+    def mlp(self, ws, m, st):
+        return self.lib.q35mm_mlp(*ws, self.x, 1e-6, m, self.x, st), self.take()
+
+    def capture(self, st, on=True):
+        self.lib.stub_capture(st, int(on))
+
+
+@pytest.fixture
+def lib(stub_path):
+    lb = Lib(stub_path)
+    yield lb
+    lb.lib.stub_fail_malloc(C.c_size_t(-1))
+    for s in (None, S, T, U):
+        lb.capture(s, False)
+    lb.lib.q35mm_shutdown()
+    lb.take()
+
+
+def kinds(rec):
+    return [r[0] for r in rec]
+
+
+def pointers(rec):
+    """Scratch addresses a call's launches carry."""
+    return {v for _, f, _ in rec for k, v in f.items() if k in ("xs", "xf", "ws", "xb", "cnt") and v != "(nil)"}
+
+
+def test_eager_batch(lib):
+    """What the other tests build on: outside capture 24 tokens are a batch."""
+    w = lib.weight(300, 1024)
+    rc, rec = lib.matmul(w, 24, S)
+    assert rc == 0 and [k for k in kinds(rec) if k in ("split", "batch", "rows")] == ["split", "batch"]
+
+
+@pytest.mark.parametrize("m", [9, 24, 63])
+def test_captured_matmul_carries_no_scratch(lib, m):
+    """A stream with scratch of its own, warmed at the same size: two graphs
+    of the call hold no memory in common, so they may be replayed at once."""
+    w = lib.weight(300, 5120)
+    assert lib.matmul(w, m, S)[0] == 0
+    assert lib.matmul(w, 512, S)[0] == 0
+    lib.capture(S)
+    for _ in range(2):
+        rc, rec = lib.matmul(w, m, S)
+        assert rc == 0 and kinds(rec) == ["rows"] * ((m + 7) // 8) and not pointers(rec)
+
+
+@pytest.mark.parametrize("m", [9, 24])
+def test_captured_mlp_carries_only_its_workspace(lib, m):
+    """The MLP block's graph holds the block's own intermediates, as it did
+    in groups of eight tokens, and none of the scratch matmuls use."""
+    ws = [lib.weight(1664, 5120), lib.weight(1664, 5120), lib.weight(5120, 1664)]
+    assert lib.mlp(ws, m, S)[0] == 0
+    lib.capture(S)
+    rc, rec = lib.mlp(ws, m, S)
+    n = (m + 7) // 8
+    assert rc == 0 and kinds(rec) == ["rmsnorm"] + ["pair"] * n + ["rows"] * n and not pointers(rec)

@@ -132,3 +132,40 @@ def test_batch_capture(q, wl, gpu):
             torch.cuda.synchronize()
             _same_bits(Y, want)
     w.free()
+
+
+def test_graphs_replayed_at_once(q, wl, gpu):
+    """Two graphs of matmuls captured on one stream that has run the same
+    calls, replayed on two other streams beside eager calls on the first:
+    each gives its own bits."""
+    import torch
+    w = q.Weight(*wl.gen_weight(14, 5120, 5120))
+    Xs = [torch.from_numpy(wl.gen_act(15 + i, 40, 5120)).to(gpu) for i in range(3)]
+    want = [_rows_of_small_calls(q, [w], X, gpu)[0] for X in Xs]
+    Ys = [torch.zeros((40, 5120), device=gpu) for _ in range(3)]
+    s, other = torch.cuda.Stream(), [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        q.matmul(w, Xs[2], Ys[2])
+    torch.cuda.synchronize()
+    gs = []
+    for X, Y in zip(Xs[:2], Ys):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            q.matmul(w, X, Y)
+        gs.append(g)
+    for _ in range(3):
+        for Y in Ys:
+            Y.zero_()
+        torch.cuda.synchronize()
+        for _ in range(10):
+            for g, o in zip(gs, other):
+                with torch.cuda.stream(o):
+                    g.replay()
+            with torch.cuda.stream(s):
+                q.matmul(w, Xs[2], Ys[2])
+        torch.cuda.synchronize()
+        for Y, R in zip(Ys, want):
+            _same_bits(Y, R)
+    q.stream_release(s.cuda_stream)
+    w.free()
