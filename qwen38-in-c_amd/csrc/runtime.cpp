@@ -522,9 +522,8 @@ int run_gemv_group(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
 // Batched decode (gemv_batch.hip) of row-split weights: scratch for passes
 // of mp tokens over weights of up to kb K blocks and nb row groups in all.
 // xs and xf share the GEMM's activation buffer.  kNoRoom, with nothing
-// launched, when there is no scratch for it (the fixed scratch of an
-// allocation-free call), and the caller takes the launches of eight tokens,
-// which need none and give the same bits.
+// launched, when there is no scratch for it, and the caller takes the
+// launches of eight tokens, which need none and give the same bits.
 constexpr int kNoRoom = -1001;   // internal
 
 // Whether m tokens of row-split weights go as one batch.  From 17 tokens on
@@ -540,12 +539,16 @@ constexpr int kNoRoom = -1001;   // internal
 constexpr uint32_t kBatchMinKb = 28, kBatchMinKbMlp = 33;
 bool batch_pays(uint32_t m, uint32_t kb, uint32_t min_kb) { return m > 2 * kGemvMaxM || (m > kGemvMaxM && kb >= min_kb); }
 
-// Whether calls on st may use the batch's scratch.  Not in a graph capture:
-// a graph may be replayed on any stream, beside eager calls on the captured
-// one and other graphs, which would overwrite that scratch; the launches of
-// eight tokens hold none.  A stream that cannot be asked (the null stream
-// while another is captured) counts as captured.
-bool batch_allowed(hipStream_t st) {
+// Whether a call on st may use the batch's scratch.  Not an allocation-free
+// call, whose fixed scratch every stream shares: row-split weights need none
+// of it eight tokens at a time, so such calls overlap on different streams.
+// Not in a graph capture: a graph may be replayed on any stream, beside
+// eager calls on the captured one and other graphs, which would overwrite
+// that scratch; the launches of eight tokens hold none.  A stream that
+// cannot be asked (the null stream while another is captured) counts as
+// captured.
+bool batch_allowed(hipStream_t st, const Scratch *scr) {
+    if (scr && scr->fixed) return false;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs == hipStreamCaptureStatusNone;
     (void)hipGetLastError();   // or the next launch would report it
@@ -555,7 +558,6 @@ bool batch_allowed(hipStream_t st) {
 int batch_scratch(Scratch &sc, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t **xs, float **xf, float **ws) {
     const size_t ab = batch_act_bytes(mp, kb), fb = 2 * (size_t)kb * sizeof(float);   // at most two tiles
     const size_t xb = (ab + fb + 255) & ~(size_t)255, wb = batch_ws_floats(mp, nb, g_dev.rows_waves) * sizeof(float);
-    if (sc.fixed && xb + wb > kNoAllocBytes) return kNoRoom;
     uint16_t *x = nullptr;
     const int rc = scratch_gemm(sc, xb, wb, &x, ws);
     if (rc) return rc;
@@ -581,7 +583,7 @@ uint32_t batch_seg(BatchParams &p, uint32_t s, const Weight &w, float *y, const 
 
 int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const float *dX, float *const *dY,
                    hipStream_t st, float *const *resid, Scratch *scr) {
-    if (!batch_allowed(st)) return kNoRoom;
+    if (!batch_allowed(st, scr)) return kNoRoom;
     Scratch &sc = scr ? *scr : scratch_for(st);
     const uint32_t cols = w[0]->w.cols, kb = w[0]->w.kb;
     uint64_t nb = 0;
@@ -590,8 +592,7 @@ int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
     p.kb = kb;
     p.nseg = nseg;
     p.nr = g_dev.rows_waves;
-    // tokens per pass: fewer where the range sums pass ws_off's 32 bits or
-    // the fixed scratch of an allocation-free call
+    // tokens per pass: fewer where the range sums pass ws_off's 32 bits
     uint32_t mp = std::min(m, kBatchTokens);
     uint8_t *xs = nullptr;
     float *xf = nullptr;
@@ -1808,7 +1809,7 @@ int run_mlp_batch(const q35mm_weight *gate, const q35mm_weight *up, const q35mm_
     const uint32_t H = g.cols, mp = std::min(m, kBatchTokens), kb = std::max(g.kb, d.kb), nb = std::max(2 * g.nb, d.nb);
     BatchParams p{};
     p.nr = g_dev.rows_waves;
-    if (!batch_allowed(st) || batch_ws_floats(mp, nb, p.nr) > UINT32_MAX) return kNoRoom;
+    if (!batch_allowed(st, &scr) || batch_ws_floats(mp, nb, p.nr) > UINT32_MAX) return kNoRoom;
     uint8_t *xs = nullptr;
     float *xf = nullptr;
     const int rc = batch_scratch(scr, mp, kb, nb, &xs, &xf, &p.ws);

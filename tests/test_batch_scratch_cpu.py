@@ -125,3 +125,13 @@ def test_captured_mlp_carries_only_its_workspace(lib, m):
     rc, rec = lib.mlp(ws, m, S)
     n = (m + 7) // 8
     assert rc == 0 and kinds(rec) == ["rmsnorm"] + ["pair"] * n + ["rows"] * n and not pointers(rec)
+
+
+@pytest.mark.parametrize("m", [9, 24, 63])
+def test_noalloc_uses_no_shared_scratch(lib, m):
+    """Every stream's allocation-free calls share one fixed array; row-split
+    weights use none of it, so these calls may overlap on two streams."""
+    w = lib.weight(300, 5120)
+    rc = lib.lib.q35mm_matmul_noalloc(w, m, lib.x, lib.y, S)
+    rec = lib.take()
+    assert rc == 0 and kinds(rec) == ["rows"] * ((m + 7) // 8) and not pointers(rec)
