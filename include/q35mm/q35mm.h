@@ -18,7 +18,8 @@
  * Streams are hipStream_t passed as void*; NULL is HIP's null stream.
  *
  * Concurrency: scratch memory between a call's kernels (split-K partials
- * and counters, the GEMM's bf16 activations, the MLP block's intermediates)
+ * and counters, the GEMM's bf16 activations, the MLP block's intermediates,
+ * the split activations and K-range sums of 9..63 tokens)
  * is kept per stream, so calls on different streams may overlap on the GPU.
  * Calls on one stream run in order.  Host threads may call concurrently
  * (calls are serialised on a library lock while they queue work).

@@ -111,6 +111,11 @@ struct Device {
     hipStream_t stream = nullptr;
     std::unordered_map<hipStream_t, Scratch> scratch;
     Scratch *last_scratch = nullptr;   // of the most recent call outside graph capture
+    // The batched decode's scratch, one buffer per stream beside its set: no
+    // graph holds it (a set's buffers may be in a graph that replays beside
+    // eager calls), and a stream that only ran batches has no set a capture
+    // could be given.
+    std::unordered_map<hipStream_t, DevBuf> batch;
     std::vector<void *> retired;       // buffers a captured graph may still use (freed at shutdown)
     DevBuf dx, dy;    // activation staging for the host-pointer ABI
     void *up_pin[4] = {};        // pinned chunks of the file -> HBM upload ring
@@ -519,11 +524,9 @@ int run_gemv_group(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
     return Q35MM_OK;
 }
 
-// Batched decode (gemv_batch.hip) of row-split weights: scratch for passes
-// of mp tokens over weights of up to kb K blocks and nb row groups in all.
-// xs and xf share the GEMM's activation buffer.  kNoRoom, with nothing
-// launched, when there is no scratch for it, and the caller takes the
-// launches of eight tokens, which need none and give the same bits.
+// Batched decode (gemv_batch.hip) of row-split weights.  kNoRoom, with
+// nothing launched, when there is no scratch for it, and the caller takes
+// the launches of eight tokens, which need none and give the same bits.
 constexpr int kNoRoom = -1001;   // internal
 
 // Whether m tokens of row-split weights go as one batch.  From 17 tokens on
@@ -555,14 +558,17 @@ bool batch_allowed(hipStream_t st, const Scratch *scr) {
     return false;
 }
 
-int batch_scratch(Scratch &sc, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t **xs, float **xf, float **ws) {
+// Scratch for passes of mp tokens over weights of up to kb K blocks and nb
+// row groups in all.
+int batch_scratch(hipStream_t st, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t **xs, float **xf, float **ws) {
     const size_t ab = batch_act_bytes(mp, kb), fb = 2 * (size_t)kb * sizeof(float);   // at most two tiles
     const size_t xb = (ab + fb + 255) & ~(size_t)255, wb = batch_ws_floats(mp, nb, g_dev.rows_waves) * sizeof(float);
-    uint16_t *x = nullptr;
-    const int rc = scratch_gemm(sc, xb, wb, &x, ws);
+    DevBuf &b = g_dev.batch[st];
+    const int rc = grow(b, xb + wb, false);
     if (rc) return rc;
-    *xs = reinterpret_cast<uint8_t *>(x);
+    *xs = static_cast<uint8_t *>(b.ptr);
     *xf = reinterpret_cast<float *>(*xs + ab);
+    *ws = reinterpret_cast<float *>(*xs + xb);
     return Q35MM_OK;
 }
 
@@ -584,7 +590,6 @@ uint32_t batch_seg(BatchParams &p, uint32_t s, const Weight &w, float *y, const 
 int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const float *dX, float *const *dY,
                    hipStream_t st, float *const *resid, Scratch *scr) {
     if (!batch_allowed(st, scr)) return kNoRoom;
-    Scratch &sc = scr ? *scr : scratch_for(st);
     const uint32_t cols = w[0]->w.cols, kb = w[0]->w.kb;
     uint64_t nb = 0;
     for (uint32_t s = 0; s < nseg; s++) nb += w[s]->w.nb;
@@ -599,7 +604,7 @@ int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
     int rc = kNoRoom;
     for (; rc == kNoRoom && mp > kGemvMaxM; mp = mp > 32 ? 32 : mp > 16 ? 16 : 0) {
         if (batch_ws_floats(mp, 1, p.nr) * nb > UINT32_MAX) continue;
-        rc = batch_scratch(sc, mp, kb, (uint32_t)nb, &xs, &xf, &p.ws);
+        rc = batch_scratch(st, mp, kb, (uint32_t)nb, &xs, &xf, &p.ws);
         if (rc != kNoRoom) break;
     }
     if (rc) return rc;
@@ -1804,15 +1809,15 @@ int run_mlp_pair(const q35mm_weight *gate, const q35mm_weight *up, uint32_t m, c
 // product's split activations in one kernel.  Bits as above; kNoRoom as
 // batch_scratch.
 int run_mlp_batch(const q35mm_weight *gate, const q35mm_weight *up, const q35mm_weight *down, uint32_t m,
-                  const float *xn, float *dX, hipStream_t st, Scratch &scr) {
+                  const float *xn, float *dX, hipStream_t st) {
     const Weight &g = gate->w, &u = up->w, &d = down->w;
     const uint32_t H = g.cols, mp = std::min(m, kBatchTokens), kb = std::max(g.kb, d.kb), nb = std::max(2 * g.nb, d.nb);
     BatchParams p{};
     p.nr = g_dev.rows_waves;
-    if (!batch_allowed(st, &scr) || batch_ws_floats(mp, nb, p.nr) > UINT32_MAX) return kNoRoom;
+    if (!batch_allowed(st, nullptr) || batch_ws_floats(mp, nb, p.nr) > UINT32_MAX) return kNoRoom;
     uint8_t *xs = nullptr;
     float *xf = nullptr;
-    const int rc = batch_scratch(scr, mp, kb, nb, &xs, &xf, &p.ws);
+    const int rc = batch_scratch(st, mp, kb, nb, &xs, &xf, &p.ws);
     if (rc) return rc;
     p.xs = xs;
     p.xf = xf;
@@ -1880,7 +1885,7 @@ Q35MM_API int q35mm_mlp(const q35mm_weight *gate, const q35mm_weight *up, const 
             const bool norm_in = m == 1 && H <= kPairNormMaxCols && g_dev.mlp_pair == 1;
             if (!norm_in) HIP_TRY(launch_rmsnorm(dX, H, dNormW, xn, H, m, H, eps, st));
             if (batch_pays(m, gate->w.kb + down->w.kb, kBatchMinKbMlp) && uses_gemv_rows(down->w)) {
-                rc = run_mlp_batch(gate, up, down, m, xn, dX, st, scr);
+                rc = run_mlp_batch(gate, up, down, m, xn, dX, st);
                 if (rc != kNoRoom) return rc;
             }
             for (uint32_t t0 = 0; t0 < m; t0 += kGemvMaxM) {
@@ -2073,6 +2078,9 @@ Q35MM_API void q35mm_shutdown(void) {
             if (b->ptr) (void)hipFree(b->ptr);
     g_dev.scratch.clear();
     g_dev.last_scratch = nullptr;
+    for (auto &kv : g_dev.batch)
+        if (kv.second.ptr) (void)hipFree(kv.second.ptr);
+    g_dev.batch.clear();
     for (void *ptr : g_dev.retired) (void)hipFree(ptr);
     g_dev.retired.clear();
     for (DevBuf *b : {&g_dev.dx, &g_dev.dy}) {
@@ -2295,8 +2303,15 @@ Q35MM_API int q35mm_stream_release(void *stream) {
     std::lock_guard<std::recursive_mutex> lk(g_mu);
     if (g_dev.id < 0) return Q35MM_OK;
     auto it = g_dev.scratch.find(pick_stream(stream));
-    if (it == g_dev.scratch.end()) return Q35MM_OK;
+    auto bt = g_dev.batch.find(pick_stream(stream));
+    if (it == g_dev.scratch.end() && bt == g_dev.batch.end()) return Q35MM_OK;
     HIP_TRY(hipDeviceSynchronize());
+    if (bt != g_dev.batch.end()) {
+        void *ptr = bt->second.ptr;
+        g_dev.batch.erase(bt);
+        if (ptr) HIP_TRY(hipFree(ptr));
+    }
+    if (it == g_dev.scratch.end()) return Q35MM_OK;
     Scratch &s = it->second;
     for (DevBuf *b : {&s.ws, &s.cnt, &s.xb, &s.mlp}) {
         if (!b->ptr) continue;

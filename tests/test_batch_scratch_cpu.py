@@ -135,3 +135,46 @@ def test_noalloc_uses_no_shared_scratch(lib, m):
     rc = lib.lib.q35mm_matmul_noalloc(w, m, lib.x, lib.y, S)
     rec = lib.take()
     assert rc == 0 and kinds(rec) == ["rows"] * ((m + 7) // 8) and not pointers(rec)
+
+
+@pytest.mark.parametrize("what", ["matmul", "mlp"])
+def test_batch_shares_nothing_with_graphs(lib, what):
+    """A graph of a GEMM or a prefill MLP block holds its stream's scratch
+    set; row-split matmuls never wrote to it, so the graph could replay
+    beside them.  The batch's scratch is none of the graph's."""
+    ws = [lib.weight(1664, 5120), lib.weight(1664, 5120), lib.weight(5120, 1664)]
+    run = lib.matmul if what == "matmul" else lib.mlp
+    arg = ws[0] if what == "matmul" else ws
+    assert run(arg, 512, S)[0] == 0
+    lib.capture(S)
+    rc, rec = run(arg, 512, S)
+    held = pointers(rec)
+    assert rc == 0 and held
+    lib.capture(S, False)
+    rc, rec = lib.matmul(ws[0], 63, S)
+    assert rc == 0 and "batch" in kinds(rec) and not pointers(rec) & held
+
+
+def test_batch_does_not_move_the_borrowed_set(lib):
+    """A capture on a new stream borrows the set of the last call that has
+    one: batches in between, on another stream or captured, change nothing."""
+    w = lib.weight(300, 5120)
+    assert lib.matmul(w, 1, S)[0] == 0
+    lib.capture(S)
+    assert lib.matmul(w, 24, S)[0] == 0
+    lib.capture(S, False)
+    assert lib.matmul(w, 512, T)[0] == 0
+    assert lib.matmul(w, 24, U)[0] == 0
+    lib.capture(S)
+    rc, rec = lib.matmul(w, 512, S)
+    assert rc == 0 and "gemm" in kinds(rec)
+
+
+def test_batch_scratch_is_given_back(lib):
+    """q35mm_stream_release frees a stream's batch scratch."""
+    w = lib.weight(300, 5120)
+    rc, rec = lib.matmul(w, 63, S)
+    got = [ln.split()[1] for k, _, ln in rec if k == "malloc"]
+    assert rc == 0 and got
+    assert lib.lib.q35mm_stream_release(S) == 0
+    assert sorted(ln.split()[1] for k, _, ln in lib.take() if k == "free") == sorted(got)
