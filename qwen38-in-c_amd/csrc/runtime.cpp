@@ -106,6 +106,14 @@ struct Scratch {
     bool capturing = false;
 };
 
+// The batched decode's scratch of one stream.  Outgrown buffers, which
+// kernels in flight may still use, stay until the stream's release: growth
+// doubles, so together they are no larger than the current one.
+struct BatchBuf {
+    DevBuf buf;
+    std::vector<void *> old;
+};
+
 struct Device {
     int id = -1;
     hipStream_t stream = nullptr;
@@ -115,7 +123,7 @@ struct Device {
     // graph holds it (a set's buffers may be in a graph that replays beside
     // eager calls), and a stream that only ran batches has no set a capture
     // could be given.
-    std::unordered_map<hipStream_t, DevBuf> batch;
+    std::unordered_map<hipStream_t, BatchBuf> batch;
     std::vector<void *> retired;       // buffers a captured graph may still use (freed at shutdown)
     DevBuf dx, dy;    // activation staging for the host-pointer ABI
     void *up_pin[4] = {};        // pinned chunks of the file -> HBM upload ring
@@ -563,13 +571,42 @@ bool batch_allowed(hipStream_t st, const Scratch *scr) {
 int batch_scratch(hipStream_t st, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t **xs, float **xf, float **ws) {
     const size_t ab = batch_act_bytes(mp, kb), fb = 2 * (size_t)kb * sizeof(float);   // at most two tiles
     const size_t xb = (ab + fb + 255) & ~(size_t)255, wb = batch_ws_floats(mp, nb, g_dev.rows_waves) * sizeof(float);
-    DevBuf &b = g_dev.batch[st];
-    const int rc = grow(b, xb + wb, false);
-    if (rc) return rc;
+    BatchBuf &bb = g_dev.batch[st];
+    DevBuf &b = bb.buf;
+    if (b.cap < xb + wb) {
+        // No wait for the device, as these calls never had one, and no
+        // failure: eight tokens need no memory.  The relaxed mode lets the
+        // thread allocate while another thread captures.
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+        void *ptr = nullptr;
+        const size_t cap = (std::max(xb + wb, 2 * b.cap) + 4095) & ~(size_t)4095;
+        const hipError_t e = hipMalloc(&ptr, cap);
+        HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+        if (e != hipSuccess) {
+            (void)hipGetLastError();   // or the next launch would report it
+            return kNoRoom;
+        }
+        if (b.ptr) bb.old.push_back(b.ptr);
+        b.ptr = ptr;
+        b.cap = cap;
+    }
     *xs = static_cast<uint8_t *>(b.ptr);
     *xf = reinterpret_cast<float *>(*xs + ab);
     *ws = reinterpret_cast<float *>(*xs + xb);
     return Q35MM_OK;
+}
+
+// Frees a stream's batch scratch once its work is done; the first error.
+hipError_t free_batch(BatchBuf &b) {
+    hipError_t e = hipSuccess;
+    b.old.push_back(b.buf.ptr);
+    for (void *ptr : b.old) {
+        const hipError_t f = ptr ? hipFree(ptr) : hipSuccess;
+        if (e == hipSuccess) e = f;
+    }
+    b = BatchBuf();
+    return e;
 }
 
 // One weight of a batched pass of p.m tokens; returns the next one's ws_off.
@@ -597,7 +634,8 @@ int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
     p.kb = kb;
     p.nseg = nseg;
     p.nr = g_dev.rows_waves;
-    // tokens per pass: fewer where the range sums pass ws_off's 32 bits
+    // tokens per pass: fewer where the range sums pass ws_off's 32 bits or
+    // there is no memory for them
     uint32_t mp = std::min(m, kBatchTokens);
     uint8_t *xs = nullptr;
     float *xf = nullptr;
@@ -2078,8 +2116,7 @@ Q35MM_API void q35mm_shutdown(void) {
             if (b->ptr) (void)hipFree(b->ptr);
     g_dev.scratch.clear();
     g_dev.last_scratch = nullptr;
-    for (auto &kv : g_dev.batch)
-        if (kv.second.ptr) (void)hipFree(kv.second.ptr);
+    for (auto &kv : g_dev.batch) (void)free_batch(kv.second);
     g_dev.batch.clear();
     for (void *ptr : g_dev.retired) (void)hipFree(ptr);
     g_dev.retired.clear();
@@ -2307,9 +2344,9 @@ Q35MM_API int q35mm_stream_release(void *stream) {
     if (it == g_dev.scratch.end() && bt == g_dev.batch.end()) return Q35MM_OK;
     HIP_TRY(hipDeviceSynchronize());
     if (bt != g_dev.batch.end()) {
-        void *ptr = bt->second.ptr;
+        const hipError_t e = free_batch(bt->second);
         g_dev.batch.erase(bt);
-        if (ptr) HIP_TRY(hipFree(ptr));
+        HIP_TRY(e);
     }
     if (it == g_dev.scratch.end()) return Q35MM_OK;
     Scratch &s = it->second;

@@ -9,6 +9,7 @@
 #include <cstring>
 #include <set>
 #include <string>
+#include <utility>
 
 #include "q35mm_internal.h"
 
@@ -19,6 +20,7 @@ std::string g_log;
 std::set<void *> g_capturing;   // streams under capture
 size_t g_fail_from = SIZE_MAX;  // allocations of at least this size fail
 hipError_t g_last = hipSuccess;
+hipStreamCaptureMode g_mode = hipStreamCaptureModeGlobal;   // the calling thread's
 
 template <typename... A>
 hipError_t note(const char *fmt, A... a) {
@@ -59,8 +61,8 @@ hipError_t hipGetLastError() {
     return e;
 }
 hipError_t hipMalloc(void **p, size_t n) {
-    // while any stream is captured (in the global mode) an allocation is refused
-    if (!g_capturing.empty()) return fail(hipErrorStreamCaptureUnsupported);
+    // while any stream is captured, a thread in the global mode may not allocate
+    if (!g_capturing.empty() && g_mode == hipStreamCaptureModeGlobal) return fail(hipErrorStreamCaptureUnsupported);
     if (n >= g_fail_from) return fail(hipErrorOutOfMemory);
     *p = aligned_alloc(256, (n + 255) & ~(size_t)255);
     return note("malloc %p %zu", *p, n);
@@ -75,6 +77,7 @@ hipError_t hipHostFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { return memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemset(void *d, int v, size_t n) { return memset(d, v, n), hipSuccess; }
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode *m) { return std::swap(*m, g_mode), hipSuccess; }
 hipError_t hipDeviceSynchronize() { return note("device_sync"); }
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return *s = (hipStream_t)malloc(1), hipSuccess; }
 hipError_t hipStreamDestroy(hipStream_t s) { return free((void *)s), hipSuccess; }

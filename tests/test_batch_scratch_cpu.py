@@ -178,3 +178,49 @@ def test_batch_scratch_is_given_back(lib):
     assert rc == 0 and got
     assert lib.lib.q35mm_stream_release(S) == 0
     assert sorted(ln.split()[1] for k, _, ln in lib.take() if k == "free") == sorted(got)
+
+
+def test_no_memory_runs_eight_at_a_time(lib):
+    """Eight tokens need no memory: a batch that gets none runs as they do,
+    one that gets less in passes of 32 or 16 tokens, and neither fails."""
+    w = lib.weight(30000, 512)
+    lib.lib.stub_fail_malloc(1)
+    rc, rec = lib.matmul(w, 63, S)
+    assert rc == 0 and kinds(rec) == ["rows"] * 8
+    lib.lib.stub_fail_malloc(20 << 20)          # 30 MB of range sums at 63 tokens, 15 at 32
+    rc, rec = lib.matmul(w, 63, S)
+    assert rc == 0 and [f["m"] for k, f, _ in rec if k == "batch"] == ["32", "31"]
+    ws = [lib.weight(1664, 512), lib.weight(1664, 512), lib.weight(512, 1664)]
+    assert lib.mlp(ws, 1, U)[0] == 0 and lib.mlp(ws, 24, U)[0] == 0
+    assert lib.lib.q35mm_stream_release(U) == 0
+    assert lib.mlp(ws, 1, U)[0] == 0 and lib.lib.q35mm_mlp(*ws, lib.x, 1e-6, 64, lib.x, U) == 0   # its workspace
+    lib.take()
+    lib.lib.stub_fail_malloc(1)
+    rc, rec = lib.mlp(ws, 24, U)
+    assert rc == 0 and kinds(rec) == ["rmsnorm"] + ["pair"] * 3 + ["rows"] * 3
+
+
+def test_growth_neither_waits_nor_frees(lib):
+    """Matmuls of 9..63 tokens never waited for the device; kernels in flight
+    may still use the smaller buffer, which stays until the stream's release."""
+    w = lib.weight(30000, 512)
+    recs = []
+    for m in (9, 24, 63, 63):
+        rc, rec = lib.matmul(w, m, S)
+        assert rc == 0
+        recs += rec
+    got = [ln.split()[1] for k, _, ln in recs if k == "malloc"]
+    assert len(got) >= 2 and not {"device_sync", "free"} & set(kinds(recs))
+    assert lib.lib.q35mm_stream_release(S) == 0
+    assert sorted(ln.split()[1] for k, _, ln in lib.take() if k == "free") == sorted(got)
+
+
+def test_beside_another_threads_capture(lib):
+    """A capture on another stream does not refuse a first batch: 24 tokens
+    on S while T is captured."""
+    w = lib.weight(300, 5120)
+    lib.capture(T)
+    rc, rec = lib.matmul(w, 24, S)
+    assert rc == 0 and "batch" in kinds(rec)
+    rc, rec = lib.matmul(w, 24, None)           # the null stream cannot be asked
+    assert rc == 0 and kinds(rec) == ["rows"] * 3
