@@ -557,9 +557,10 @@ bool batch_pays(uint32_t m, uint32_t kb, uint32_t min_kb) { return m > 2 * kGemv
 // eager calls on the captured one and other graphs, which would overwrite
 // that scratch; the launches of eight tokens hold none.  A stream that
 // cannot be asked (the null stream while another is captured) counts as
-// captured.
+// captured.  hipStreamPerThread is another stream in each thread under one
+// handle, so no scratch can be kept for it.
 bool batch_allowed(hipStream_t st, const Scratch *scr) {
-    if (scr && scr->fixed) return false;
+    if ((scr && scr->fixed) || st == hipStreamPerThread) return false;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs == hipStreamCaptureStatusNone;
     (void)hipGetLastError();   // or the next launch would report it

@@ -224,3 +224,11 @@ def test_beside_another_threads_capture(lib):
     assert rc == 0 and "batch" in kinds(rec)
     rc, rec = lib.matmul(w, 24, None)           # the null stream cannot be asked
     assert rc == 0 and kinds(rec) == ["rows"] * 3
+
+
+def test_per_thread_stream_is_not_one_stream(lib):
+    """hipStreamPerThread names another stream in each host thread: nothing
+    may be kept under that handle."""
+    w = lib.weight(300, 5120)
+    rc, rec = lib.matmul(w, 24, 2)
+    assert rc == 0 and kinds(rec) == ["rows"] * 3
