@@ -156,10 +156,11 @@ __global__ __launch_bounds__(16 * T) void split_act_kernel(const float *__restri
 // without its fp32 rows in between.  One workgroup per token tile and K block
 // of the next weight, one thread per token and eight columns, columns fastest
 // (the range sums, 8 x 4 bytes an output, outweigh the 6 written).
-template <uint32_t T, uint32_t NR>
+template <uint32_t T>
 __global__ __launch_bounds__(16 * T) void batch_swiglu_kernel(BatchParams p, uint32_t kb_total, uint8_t *__restrict__ xs,
                                                               float *__restrict__ xf) {
     using Geo = BatchGeo<T>;
+    constexpr uint32_t NR = kPairWaves;
     const uint32_t kb = blockIdx.x % kb_total, tile = blockIdx.x / kb_total;
     const uint32_t u = threadIdx.x & 15, tt = threadIdx.x >> 4, t = tile * T + tt, c = kb * kBlock + u * 8;
     const uint32_t rows = p.seg[0].rows;
@@ -436,14 +437,11 @@ hipError_t launch_gemv_batch(const BatchParams &pin, bool combine, hipStream_t s
 hipError_t launch_batch_swiglu(const BatchParams &p, uint32_t kb, uint8_t *xs, float *xf, hipStream_t stream) {
     const GemvSeg &g = p.seg[0], &u = p.seg[1];
     if (p.m == 0 || p.nseg != 2 || g.rows != u.rows || g.nb != u.nb || kb != g.nb || (p.tile != 16 && p.tile != 32) ||
-        (p.nr != 4 && p.nr != 8))
+        p.nr != kPairWaves)
         return hipErrorInvalidValue;
     const uint32_t T = p.tile;
     const dim3 grid((p.m + T - 1) / T * kb);
-    using Kernel = void (*)(BatchParams, uint32_t, uint8_t *, float *);
-    const Kernel k = T == 16 ? (p.nr == 4 ? batch_swiglu_kernel<16, 4> : batch_swiglu_kernel<16, 8>)
-                             : (p.nr == 4 ? batch_swiglu_kernel<32, 4> : batch_swiglu_kernel<32, 8>);
-    hipLaunchKernelGGL(k, grid, dim3(16 * T), 0, stream, p, kb, xs, xf);
+    hipLaunchKernelGGL((T == 16 ? batch_swiglu_kernel<16> : batch_swiglu_kernel<32>), grid, dim3(16 * T), 0, stream, p, kb, xs, xf);
     return hipGetLastError();
 }
 

@@ -342,17 +342,17 @@ RowsKernel rows_kernel(uint32_t depth, uint32_t vec_mt) {
 }
 using PairKernel = void (*)(GemvParams);
 PairKernel pair_kernel(bool norm, uint32_t depth, uint32_t vec_mt) {
-#define Q35_PK(D)                                                                                       \
-    {gemv_rows_kernel<false, 1, D, 4, kRowsPair>, gemv_rows_kernel<false, 2, D, 4, kRowsPair>,          \
-     gemv_rows_kernel<false, 4, D, 4, kRowsPair>, gemv_rows_kernel<false, 8, D, 4, kRowsPair>,          \
-     gemv_rows_kernel<true, 1, D, 4, kRowsPair>,  gemv_rows_kernel<true, 2, D, 4, kRowsPair>,           \
-     gemv_rows_kernel<true, 4, D, 4, kRowsPair>,  gemv_rows_kernel<true, 8, D, 4, kRowsPair>}
+#define Q35_PK(D) \
+    {gemv_rows_kernel<false, 1, D, kPairWaves, kRowsPair>, gemv_rows_kernel<false, 2, D, kPairWaves, kRowsPair>, \
+     gemv_rows_kernel<false, 4, D, kPairWaves, kRowsPair>, gemv_rows_kernel<false, 8, D, kPairWaves, kRowsPair>, \
+     gemv_rows_kernel<true, 1, D, kPairWaves, kRowsPair>,  gemv_rows_kernel<true, 2, D, kPairWaves, kRowsPair>, \
+     gemv_rows_kernel<true, 4, D, kPairWaves, kRowsPair>,  gemv_rows_kernel<true, 8, D, kPairWaves, kRowsPair>}
     static const PairKernel k[2][8] = {Q35_PK(2), Q35_PK(3)};
 #undef Q35_PK
-    static const PairKernel kn[2][2] = {{gemv_rows_kernel<false, 1, 2, 4, kRowsPairNorm>,
-                                         gemv_rows_kernel<true, 1, 2, 4, kRowsPairNorm>},
-                                        {gemv_rows_kernel<false, 1, 3, 4, kRowsPairNorm>,
-                                         gemv_rows_kernel<true, 1, 3, 4, kRowsPairNorm>}};
+    static const PairKernel kn[2][2] = {{gemv_rows_kernel<false, 1, 2, kPairWaves, kRowsPairNorm>,
+                                         gemv_rows_kernel<true, 1, 2, kPairWaves, kRowsPairNorm>},
+                                        {gemv_rows_kernel<false, 1, 3, kPairWaves, kRowsPairNorm>,
+                                         gemv_rows_kernel<true, 1, 3, kPairWaves, kRowsPairNorm>}};
     return norm ? kn[depth - 2][vec_mt >> 2] : k[depth - 2][vec_mt];
 }
 }  // namespace
@@ -360,12 +360,12 @@ PairKernel pair_kernel(bool norm, uint32_t depth, uint32_t vec_mt) {
 hipError_t launch_gemv_pair(const GemvParams &pin, bool norm, uint32_t cus, hipStream_t stream) {
     GemvParams p = pin;
     const GemvSeg &g = p.seg[0], &u = p.seg[1];
-    if (p.xmode != kXPlain || p.m == 0 || p.m > kGemvMaxM || !gemv_rows_shape(p.kb, 4) || p.nseg != 2 ||
+    if (p.xmode != kXPlain || p.m == 0 || p.m > kGemvMaxM || !gemv_rows_shape(p.kb, kPairWaves) || p.nseg != 2 ||
         g.rows != u.rows || g.nb != u.nb || g.rows == 0 || g.cta_begin != 0)
         return hipErrorInvalidValue;
     if (norm && (p.m != 1 || p.k > kPairNormMaxCols || !p.norm_w)) return hipErrorInvalidValue;
     p.nctas = (g.rows + kPairRows - 1) / kPairRows;
-    size_t lds = 4 * (size_t)gemv_rows_wave_lds(p.m);
+    size_t lds = kPairWaves * (size_t)gemv_rows_wave_lds(p.m);
     if (norm) lds += 8 * pair_norm_stride(p.k) * sizeof(float);   // the squares of x, lane-major
     const uint32_t mt = p.m <= 1 ? 0 : p.m <= 2 ? 1 : p.m <= 4 ? 2 : 3;
     const uint32_t depth = p.m <= 2 && p.nctas <= cus ? kRsDepthLong : kRsDepthShort;
@@ -382,7 +382,7 @@ hipError_t launch_gemv_pair(const GemvParams &pin, bool norm, uint32_t cus, hipS
                 }
         attr_set = true;
     }
-    hipLaunchKernelGGL(k, dim3(p.nctas), dim3(256), lds, stream, p);
+    hipLaunchKernelGGL(k, dim3(p.nctas), dim3(64 * kPairWaves), lds, stream, p);
     return hipGetLastError();
 }
 

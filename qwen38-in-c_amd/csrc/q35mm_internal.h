@@ -143,6 +143,7 @@ hipError_t launch_gemv_rows(const GemvParams &p, uint32_t cus, uint32_t waves, u
 // one token, k <= kPairNormMaxCols: every workgroup forms the row's scale).
 constexpr uint32_t kRowsPlain = 0, kRowsPair = 1, kRowsPairNorm = 2;
 constexpr uint32_t kPairRows = 16;
+constexpr uint32_t kPairWaves = 4;   // K ranges of gate and up, whatever Q35MM_ROWS_WAVES says
 constexpr uint32_t kPairNormMaxCols = 8192;
 // Floats per lane row of the fused RMSNorm's squares in LDS ([8][stride]):
 // k/8 rounded up to whole float4, + 4 to spread the eight rows over banks.
@@ -163,7 +164,7 @@ struct BatchParams {
     const float *xf;     // scale factor per token tile and K block
     float *ws;           // range sums, segment s at ws_off: [nr][m][nb*128]
     uint32_t m, kb, nseg;
-    uint32_t nr;         // K ranges: the row-split GEMV's wavefronts (4 or 8)
+    uint32_t nr;         // K ranges: the row-split GEMV's wavefronts (4 or 8; kPairWaves for gate and up)
     uint32_t tile;       // tokens per tile (batch_tile), 16 or 32
     uint32_t groups, tiles;   // set by the launch
 };

@@ -1845,15 +1845,16 @@ int run_mlp_pair(const q35mm_weight *gate, const q35mm_weight *up, uint32_t m, c
 
 // x += down(silu(xn @ gate^T) * (xn @ up^T)) for more than kGemvMaxM tokens
 // of row-split weights: the gate and up products' range sums become the down
-// product's split activations in one kernel.  Bits as above; kNoRoom as
-// batch_scratch.
+// product's split activations in one kernel.  The bits of run_mlp_pair and
+// the down GEMV; kNoRoom as batch_scratch.
 int run_mlp_batch(const q35mm_weight *gate, const q35mm_weight *up, const q35mm_weight *down, uint32_t m,
                   const float *xn, float *dX, hipStream_t st) {
     const Weight &g = gate->w, &u = up->w, &d = down->w;
     const uint32_t H = g.cols, mp = std::min(m, kBatchTokens), kb = std::max(g.kb, d.kb), nb = std::max(2 * g.nb, d.nb);
     BatchParams p{};
-    p.nr = g_dev.rows_waves;
-    if (!batch_allowed(st, nullptr) || batch_ws_floats(mp, nb, p.nr) > UINT32_MAX) return kNoRoom;
+    const uint32_t dr = g_dev.rows_waves;   // K ranges of down; gate and up have the paired kernel's
+    static_assert(kPairWaves <= 4, "the scratch is sized by down's ranges");
+    if (!batch_allowed(st, nullptr) || batch_ws_floats(mp, nb, dr) > UINT32_MAX) return kNoRoom;
     uint8_t *xs = nullptr;
     float *xf = nullptr;
     const int rc = batch_scratch(st, mp, kb, nb, &xs, &xf, &p.ws);
@@ -1864,6 +1865,7 @@ int run_mlp_batch(const q35mm_weight *gate, const q35mm_weight *up, const q35mm_
         float *const x = dX + (size_t)t0 * H;
         p.m = std::min(mp, m - t0);
         p.kb = g.kb;
+        p.nr = kPairWaves;
         p.nseg = 2;
         batch_seg(p, 1, u, nullptr, nullptr, batch_seg(p, 0, g, nullptr, nullptr, 0));
         p.tile = batch_tile(p.m);
@@ -1871,6 +1873,7 @@ int run_mlp_batch(const q35mm_weight *gate, const q35mm_weight *up, const q35mm_
         HIP_TRY(launch_gemv_batch(p, false, st));
         HIP_TRY(launch_batch_swiglu(p, d.kb, xs, xf, st));
         p.kb = d.kb;
+        p.nr = dr;
         p.nseg = 1;
         batch_seg(p, 0, d, x, x, 0);
         HIP_TRY(launch_gemv_batch(p, true, st));

@@ -232,3 +232,20 @@ def test_per_thread_stream_is_not_one_stream(lib):
     w = lib.weight(300, 5120)
     rc, rec = lib.matmul(w, 24, 2)
     assert rc == 0 and kinds(rec) == ["rows"] * 3
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+def test_mlp_ranges_are_the_paired_kernels(stub_path, monkeypatch, waves):
+    """Gate and up of one to eight tokens are summed over four K ranges
+    whatever Q35MM_ROWS_WAVES says, down over that many: the batch's too."""
+    monkeypatch.setenv("Q35MM_ROWS_WAVES", str(waves))
+    lb = Lib(stub_path)
+    ws = [lb.weight(1664, 5120), lb.weight(1664, 5120), lb.weight(5120, 1664)]
+    seen = {}
+    for m in (8, 24):
+        rc, rec = lb.mlp(ws, m, S)
+        assert rc == 0
+        seen[m] = [(k, f["nr"]) for k, f, _ in rec if "nr" in f]
+    lb.lib.q35mm_shutdown()
+    assert seen[8] == [("pair", "4"), ("rows", str(waves))]
+    assert seen[24] == [("batch", "4"), ("batch_swiglu", "4"), ("batch", str(waves))]

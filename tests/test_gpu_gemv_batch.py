@@ -8,8 +8,14 @@ turn of the three-deep ring of each length), partial blocks both ways, both
 work splits (few and many row groups), several weights, values of any
 magnitude.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
+
+from conftest import ROOT
 
 pytestmark = pytest.mark.gpu
 
@@ -169,3 +175,43 @@ def test_graphs_replayed_at_once(q, wl, gpu):
             _same_bits(Y, R)
     q.stream_release(s.cuda_stream)
     w.free()
+
+
+def test_eight_ranges_keep_the_bits():
+    """Q35MM_ROWS_WAVES=8 (read when the library starts, so in a process of
+    its own): the batch sums eight K ranges as one to eight tokens do, the
+    MLP block's gate and up four."""
+    code = r"""
+import sys, numpy as np, torch
+sys.path.insert(0, %r)
+import q35mm as q, workload as wl
+gpu = torch.device("cuda:0")
+def same(a, b):
+    assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+for m, k, n in ((9, 3600, 200), (24, 1032, 300), (63, 5120, 129)):
+    print("matmul", m, k, n, flush=True)
+    w = q.Weight(*wl.gen_weight(k, n, k))
+    X = torch.from_numpy(wl.gen_act(m, m, k)).to(gpu)
+    Y, R = torch.empty((m, n), device=gpu), torch.empty((m, n), device=gpu)
+    q.matmul(w, X, Y)
+    for t in range(m):
+        q.matmul(w, X[t:t + 1], R[t:t + 1])
+    same(Y, R)
+for m, H, I in ((17, 2048, 1664), (40, 1032, 1100)):
+    print("mlp", m, H, I, flush=True)
+    ws = [q.Weight(*wl.gen_weight(H + i, *s)) for i, s in enumerate(((I, H), (I, H), (H, I)))]
+    nw = torch.zeros(H, device=gpu)
+    X = torch.from_numpy(wl.gen_act(m, m, H)).to(gpu)
+    R = X.clone()
+    for t in range(0, m, 8):
+        part = R[t:t + 8].clone()
+        q.mlp(*ws, nw, part)
+        R[t:t + 8] = part
+    q.mlp(*ws, nw, X)
+    same(X, R)
+print("done")
+""" % os.path.join(ROOT, "qwen38-in-c_amd")
+    out = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, Q35MM_ROWS_WAVES="8"),
+                         capture_output=True, text=True, timeout=110)
+    print(out.stdout, flush=True)
+    assert out.returncode == 0 and out.stdout.rstrip().endswith("done"), out.stdout + out.stderr[-2000:]
