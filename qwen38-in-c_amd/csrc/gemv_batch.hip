@@ -235,8 +235,9 @@ void gemv_batch_kernel(BatchParams p) {
 
     // ---- weight and activation streams: stage s is issued, activations
     // first, at the end of stage s - 4 and waited for at the end of stage
-    // s - 1.  Loads are unconditional (stages past the end read the last one
-    // again), so that wait is static: everything but the two newest ----
+    // s - 1.  Loads are unconditional (in a whole turn stages past the end
+    // read the last one again), so that wait is static: everything but the
+    // two newest ----
     const uint32_t ns = n * Geo::kStages;
     const uint8_t *const codes = sg.codes + ((size_t)rg * KB + k0) * kBlockBytes + wv * kSubBytes + lane * 16;
     const uint8_t *const xsrc = p.xs + ((size_t)tile * KB + k0) * Geo::kBlk;
@@ -261,8 +262,12 @@ void gemv_batch_kernel(BatchParams p) {
     };
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (uint32_t d = 0; d < kRing; d++) issue(d, d);
-    __builtin_amdgcn_sched_barrier(0);
+    for (uint32_t d = 0; d < kRing; d++) {
+        issue(d, d);
+        // stage by stage, as the waits count them (left to the compiler, two
+        // weight loads of stage 0 went last, and every turn drained the ring)
+        __builtin_amdgcn_sched_barrier(0);
+    }
     if (threadIdx.x < n) tab[threadIdx.x] = sc;
 
     const uint32_t hh = lane >> 5, mrow = lane & 31;
@@ -297,8 +302,11 @@ void gemv_batch_kernel(BatchParams p) {
     for (uint32_t o = 0; o < Geo::kOps; o++) read_a(0, 0, o);
     cvt_b(0, 0, 0);
     cvt_b(0, 0, 1);
-    auto step = [&](auto dc, uint32_t s) {   // stage s of the range, in ring slot d = s % kRing
+    // Stage s of the range, in ring slot d = s % kRing; tail >= 0: step tail
+    // of the last, part turn, which issues nothing.
+    auto step = [&](auto dc, uint32_t s, auto tc) {
         constexpr uint32_t d = decltype(dc)::value, dn = (d + 1) % kRing;
+        constexpr int tail = decltype(tc)::value;
         constexpr uint32_t blk = d / Geo::kStages % 2;   // the K block's half of part
         if constexpr (d % Geo::kStages == 0) {
             sc_prev = sc_cur;
@@ -308,10 +316,13 @@ void gemv_batch_kernel(BatchParams p) {
         for (uint32_t i = 0; i < kSteps; i++) {
             if (i == kSteps - 1) {
                 // this wavefront has read all of stage s, whose slot the
-                // copies take, and stage s+1 has landed; then all have
-                __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((kRing - 2) * kStageLoads));
+                // copies take, and stage s+1 has landed; then all have.
+                // (Without an issue each step leaves one stage fewer in
+                // flight: loads nobody uses would not be there to count.)
+                __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0((kRing - 2 - (tail < 0 ? 0 : tail)) * kStageLoads));
                 __builtin_amdgcn_s_barrier();
-                issue(d, s + kRing);
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (tail < 0) issue(d, s + kRing);
             }
             __builtin_amdgcn_sched_barrier(0);
             const uint32_t ns_slot = i == kSteps - 1 ? dn : d, ni = (i + 1) % kSteps;
@@ -335,18 +346,23 @@ void gemv_batch_kernel(BatchParams p) {
     // flight, also lead back to its start, and each turn would wait for the
     // newest weights.
     using std::integral_constant;
+    const integral_constant<uint32_t, 0> d0;
+    const integral_constant<uint32_t, 1> d1;
+    const integral_constant<uint32_t, 2> d2;
+    const integral_constant<uint32_t, 3> d3;
+    const integral_constant<int, -1> turn;
     uint32_t s = 0;
     for (; s + kRing <= ns; s += kRing) {
-        step(integral_constant<uint32_t, 0>{}, s);
-        step(integral_constant<uint32_t, 1>{}, s + 1);
-        step(integral_constant<uint32_t, 2>{}, s + 2);
-        step(integral_constant<uint32_t, 3>{}, s + 3);
+        step(d0, s, turn);
+        step(d1, s + 1, turn);
+        step(d2, s + 2, turn);
+        step(d3, s + 3, turn);
     }
     static_assert(kRing == 4, "steps of a turn");
-    if (s < ns) step(integral_constant<uint32_t, 0>{}, s);
-    if (s + 1 < ns) step(integral_constant<uint32_t, 1>{}, s + 1);
+    if (s < ns) step(d0, s, integral_constant<int, 0>{});
+    if (s + 1 < ns) step(d1, s + 1, integral_constant<int, 1>{});
     if constexpr (Geo::kStages == 1)
-        if (s + 2 < ns) step(integral_constant<uint32_t, 2>{}, s + 2);
+        if (s + 2 < ns) step(d2, s + 2, integral_constant<int, 2>{});
     __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(0));   // no copy outlives the loop
 #pragma unroll
     for (uint32_t x = 0; x < kSums; x++) {   // the last K block's sums
