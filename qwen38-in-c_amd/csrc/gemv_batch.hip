@@ -41,7 +41,8 @@
 // Bits.  The decode GEMV sums each of its K ranges block by block (one fmaf
 // with the block's scale per block and part), adds the three parts, then the
 // ranges in order.  Every step is kept: MFMA A rows only select tokens and
-// parts, so which rows they sit in does not change a sum.
+// parts, so which rows they sit in does not change a sum.  (Wide values shift
+// a K block for the eight tokens of their launch there, their eight here.)
 #include <algorithm>
 #include <type_traits>
 
@@ -58,6 +59,8 @@ typedef __attribute__((address_space(3))) uint8_t lds_u8;
 // whole one at 16.
 constexpr uint32_t kRing = 4;        // stages of activations in LDS, of weights in registers
 constexpr uint32_t kPieces = 3;      // 1 KiB activation copies per wavefront and stage
+// Scale factors of a range, at most 4 per K block (32 tokens), 2 at 16
+constexpr uint32_t kTabFloats = 4 * ((kGemvRsMaxKb + 3) / 4);
 
 // Per K block: 8 MFMA steps (chunk j < 4, half q < 2), each an MFMA's A
 // operand after another as its lanes read them (lane * 16: consecutive, or
@@ -76,6 +79,7 @@ struct BatchGeo {
     // of 16 tokens and, in a second MFMA, part 2
     static constexpr uint32_t kOps = T == 32 ? 3 : 2;
     static constexpr uint32_t kRegs = T / 2;          // token rows per lane and part
+    static constexpr uint32_t kGroups = T / kGemvMaxM;   // of eight tokens, each shifted by itself
     static_assert(kStage == 4 * kPieces * kChunkBytes, "four wavefronts copy a stage");
     static __device__ __forceinline__ uint32_t part_off(uint32_t h, uint32_t part, uint32_t t) {
         if constexpr (T == 32) return part * 1024 + h * 512 + t * 16;
@@ -121,9 +125,35 @@ __device__ __forceinline__ void store_split(uint8_t *blk, uint32_t u, uint32_t t
     *reinterpret_cast<u32x4_t *>(d + Geo::part_off(h, 2, t)) = u32x4_t{p2[0], p2[1], p2[2], p2[3]};
 }
 
+// Bit g: one of the workgroup's threads with tokens 8g..8g+7 of the tile (tt:
+// a thread's token) holds a wide value.  The row-split GEMV shifts a K block
+// for the eight tokens of a launch, so each eight here have a factor of
+// their own: values below 2^-62 of the tile's other tokens keep their bits.
+template <uint32_t T>
+__device__ __forceinline__ uint32_t wide_groups(bool wide, uint32_t tt) {
+    __shared__ uint32_t found[T / 4];   // per wavefront
+    uint32_t bits = 0;
+#pragma unroll
+    for (uint32_t g = 0; g < BatchGeo<T>::kGroups; g++)
+        bits |= __builtin_amdgcn_ballot_w64(wide && tt / kGemvMaxM == g) != 0 ? 1u << g : 0u;
+    if ((threadIdx.x & 63) == 0) found[threadIdx.x >> 6] = bits;
+    __syncthreads();
+    bits = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < T / 4; w++) bits |= found[w];
+    return bits;
+}
+
+// The scale factors of a tile's K block, its groups of eight tokens in order.
+template <uint32_t T>
+__device__ __forceinline__ void store_factors(float *__restrict__ xf, uint32_t groups) {
+    constexpr uint32_t kG = BatchGeo<T>::kGroups;
+    if (threadIdx.x < kG) xf[(size_t)blockIdx.x * kG + threadIdx.x] = groups >> threadIdx.x & 1 ? kActUnshift : 1.0f;
+}
+
 // X fp32 [m][ldx] -> split A operands (BatchGeo's layout per token tile and
-// K block) and one scale factor per tile and K block: 1, or kActUnshift for a
-// block that holds a wide value and was staged times kActShift.  Tokens past
+// K block) and one scale factor per tile, K block and eight tokens: 1, or
+// kActUnshift if they hold a wide value and were staged times kActShift.  Tokens past
 // m and columns past k are zeros.  One workgroup per tile and K block; a
 // thread splits eight columns of a token.
 template <uint32_t T, bool VEC>
@@ -146,9 +176,9 @@ __global__ __launch_bounds__(16 * T) void split_act_kernel(const float *__restri
 #pragma unroll
     for (uint32_t e = 0; e < 8; e++)
         if (t >= m || c + e >= k) v[e] = 0.0f;
-    const bool wide = __syncthreads_or(max_abs(v) >= kActWide) != 0;
-    if (threadIdx.x == 0) xf[blockIdx.x] = wide ? kActUnshift : 1.0f;
-    store_split<T>(xs + (size_t)blockIdx.x * BatchGeo<T>::kBlk, u, tt, v, wide);
+    const uint32_t groups = wide_groups<T>(max_abs(v) >= kActWide, tt);
+    store_factors<T>(xf, groups);
+    store_split<T>(xs + (size_t)blockIdx.x * BatchGeo<T>::kBlk, u, tt, v, groups >> tt / kGemvMaxM & 1);
 }
 
 // silu(gate) * up of the range sums of two weights (segments 0 and 1), split
@@ -194,9 +224,9 @@ __global__ __launch_bounds__(16 * T) void batch_swiglu_kernel(BatchParams p, uin
 #pragma unroll
         for (uint32_t e = 0; e < 8; e++) v[e] = c + e < rows ? swiglu1(sum[0][e], sum[1][e]) : 0.0f;
     }
-    const bool wide = __syncthreads_or(max_abs(v) >= kActWide) != 0;
-    if (threadIdx.x == 0) xf[blockIdx.x] = wide ? kActUnshift : 1.0f;
-    store_split<T>(xs + (size_t)blockIdx.x * Geo::kBlk, u, tt, v, wide);
+    const uint32_t groups = wide_groups<T>(max_abs(v) >= kActWide, tt);
+    store_factors<T>(xf, groups);
+    store_split<T>(xs + (size_t)blockIdx.x * Geo::kBlk, u, tt, v, groups >> tt / kGemvMaxM & 1);
 }
 
 // One K range of a 128-row group for T tokens: its sums to p.ws.
@@ -230,8 +260,10 @@ void gemv_batch_kernel(BatchParams p) {
 
     // ---- block scales, loaded before the stream so that waiting for them
     // waits for nothing else ----
-    const uint32_t kbl = k0 + min(threadIdx.x, n - 1);
-    const float sc = sg.scale[(size_t)rg * KB + kbl] * p.xf[(size_t)tile * KB + kbl];
+    // (thread i: K block i / kG, tokens 8 (i % kG) on)
+    constexpr uint32_t kG = Geo::kGroups;
+    const uint32_t kbl = k0 + min(threadIdx.x / kG, n - 1);
+    const float sc = sg.scale[(size_t)rg * KB + kbl] * p.xf[((size_t)tile * KB + kbl) * kG + threadIdx.x % kG];
 
     // ---- weight and activation streams: stage s is issued, activations
     // first, at the end of stage s - 4 and waited for at the end of stage
@@ -268,7 +300,8 @@ void gemv_batch_kernel(BatchParams p) {
         // weight loads of stage 0 went last, and every turn drained the ring)
         __builtin_amdgcn_sched_barrier(0);
     }
-    if (threadIdx.x < n) tab[threadIdx.x] = sc;
+    static_assert(kTabFloats <= 256, "one thread per factor");
+    if (threadIdx.x < n * kG) tab[threadIdx.x] = sc;
 
     const uint32_t hh = lane >> 5, mrow = lane & 31;
     const uint32_t a0 = lane * 16, a1 = 1024 + (T == 32 ? lane * 16 : hh * 256 + (mrow & 15) * 16);
@@ -285,7 +318,10 @@ void gemv_batch_kernel(BatchParams p) {
     f32x16_t acc[Geo::kOps] = {}, part[2][Geo::kOps] = {};
     const f32x16_t zero = {};
     u32x4_t aop[2][Geo::kOps], bop[2];
-    float sc_prev = 0.0f, sc_cur = 0.0f;
+    typedef float scale_t __attribute__((ext_vector_type(kG)));   // of a K block, per eight tokens
+    scale_t sc_prev = 0.0f, sc_cur = 0.0f;
+    // sum x is of rows 8 (x / 4) + 0..7 of an operand, which are tokens 8 ((x / 4) % kG) + 0..7
+    auto group = [](uint32_t x) { return x / 4 % kG; };
     auto read_a = [&](uint32_t slot, uint32_t i, uint32_t o) {
         aop[i & 1][o] = *reinterpret_cast<const u32x4_t *>(lds + slot * Geo::kStage + i * Geo::kStep +
                                                            (o == 0 ? a0 : a1 + (o - 1) * 1024));
@@ -310,7 +346,7 @@ void gemv_batch_kernel(BatchParams p) {
         constexpr uint32_t blk = d / Geo::kStages % 2;   // the K block's half of part
         if constexpr (d % Geo::kStages == 0) {
             sc_prev = sc_cur;
-            sc_cur = tab[s / Geo::kStages];
+            sc_cur = reinterpret_cast<const scale_t *>(tab)[s / Geo::kStages];
         }
 #pragma unroll
         for (uint32_t i = 0; i < kSteps; i++) {
@@ -336,7 +372,7 @@ void gemv_batch_kernel(BatchParams p) {
                 const uint32_t k = ((d % Geo::kStages) * kSteps + i) * Geo::kOps + o;
 #pragma unroll
                 for (uint32_t x = k * kSums / kSlots; x < (k + 1) * kSums / kSlots; x++)
-                    acc[x / 16][x % 16] = __builtin_fmaf(sc_prev, part[blk ^ 1][x / 16][x % 16], acc[x / 16][x % 16]);
+                    acc[x / 16][x % 16] = __builtin_fmaf(sc_prev[group(x)], part[blk ^ 1][x / 16][x % 16], acc[x / 16][x % 16]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -367,7 +403,7 @@ void gemv_batch_kernel(BatchParams p) {
 #pragma unroll
     for (uint32_t x = 0; x < kSums; x++) {   // the last K block's sums
         const float v = n & 1 ? part[0][x / 16][x % 16] : part[1][x / 16][x % 16];
-        acc[x / 16][x % 16] = __builtin_fmaf(sc_cur, v, acc[x / 16][x % 16]);
+        acc[x / 16][x % 16] = __builtin_fmaf(sc_cur[group(x)], v, acc[x / 16][x % 16]);
     }
 
     // per token row: (part 0 + part 1) + part 2
@@ -406,6 +442,8 @@ size_t batch_act_bytes(uint32_t m, uint32_t kb) {
     return (size_t)((m + 31) / 32) * kb * BatchGeo<32>::kBlk;
 }
 
+size_t batch_xf_floats(uint32_t m, uint32_t kb) { return (size_t)((m + 31) / 32) * kb * BatchGeo<32>::kGroups; }
+
 size_t batch_ws_floats(uint32_t m, uint32_t nb, uint32_t nr) { return (size_t)nr * m * nb * kBlock; }
 
 hipError_t launch_split_act(const float *x, uint32_t ldx, uint32_t m, uint32_t k, uint32_t kb, bool vec, uint32_t T,
@@ -437,7 +475,7 @@ hipError_t launch_gemv_batch(const BatchParams &pin, bool combine, hipStream_t s
         max_rows = std::max(max_rows, p.seg[s].rows);
     }
     const dim3 grid((p.groups * p.nr + 7) / 8 * 8 * p.tiles);
-    const uint32_t lds = kRing * BatchGeo<16>::kStage + kGemvRsMaxKb * sizeof(float);
+    const uint32_t lds = kRing * BatchGeo<16>::kStage + kTabFloats * sizeof(float);
     static_assert(BatchGeo<16>::kStage == BatchGeo<32>::kStage, "one ring size");
     using Kernel = void (*)(BatchParams);
     static const Kernel kernels[4] = {gemv_batch_kernel<16, false>, gemv_batch_kernel<16, true>,

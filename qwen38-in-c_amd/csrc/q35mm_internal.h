@@ -161,7 +161,7 @@ constexpr uint32_t kBatchTokens = 64;
 struct BatchParams {
     GemvSeg seg[4];
     const uint8_t *xs;   // split activations
-    const float *xf;     // scale factor per token tile and K block
+    const float *xf;     // scale factors [token tile][K block][tile / 8]
     float *ws;           // range sums, segment s at ws_off: [nr][m][nb*128]
     uint32_t m, kb, nseg;
     uint32_t nr;         // K ranges: the row-split GEMV's wavefronts (4 or 8; kPairWaves for gate and up)
@@ -170,6 +170,7 @@ struct BatchParams {
 };
 uint32_t batch_tile(uint32_t m);                                 // tokens per tile
 size_t batch_act_bytes(uint32_t m, uint32_t kb);                 // split activations, either tile
+size_t batch_xf_floats(uint32_t m, uint32_t kb);                 // their scale factors, either tile
 size_t batch_ws_floats(uint32_t m, uint32_t nb, uint32_t nr);    // range sums of one segment
 // vec: rows of x 16-byte aligned and k % 8 == 0.
 hipError_t launch_split_act(const float *x, uint32_t ldx, uint32_t m, uint32_t k, uint32_t kb, bool vec,

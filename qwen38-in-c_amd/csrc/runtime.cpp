@@ -570,7 +570,7 @@ bool batch_allowed(hipStream_t st, const Scratch *scr) {
 // Scratch for passes of mp tokens over weights of up to kb K blocks and nb
 // row groups in all.
 int batch_scratch(hipStream_t st, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t **xs, float **xf, float **ws) {
-    const size_t ab = batch_act_bytes(mp, kb), fb = 2 * (size_t)kb * sizeof(float);   // at most two tiles
+    const size_t ab = batch_act_bytes(mp, kb), fb = batch_xf_floats(mp, kb) * sizeof(float);
     const size_t xb = (ab + fb + 255) & ~(size_t)255, wb = batch_ws_floats(mp, nb, g_dev.rows_waves) * sizeof(float);
     BatchBuf &bb = g_dev.batch[st];
     DevBuf &b = bb.buf;

@@ -122,6 +122,7 @@ GemmPlan gemm_plan(uint32_t m, uint32_t ntiles, uint32_t, uint32_t, bool narrow)
 }
 uint32_t batch_tile(uint32_t m) { return m <= 16 ? 16 : 32; }
 size_t batch_act_bytes(uint32_t m, uint32_t kb) { return (size_t)((m + 31) / 32) * kb * 24576; }
+size_t batch_xf_floats(uint32_t m, uint32_t kb) { return (size_t)((m + 31) / 32) * kb * 4; }
 size_t batch_ws_floats(uint32_t m, uint32_t nb, uint32_t nr) { return (size_t)nr * m * nb * kBlock; }
 
 hipError_t launch_gemv(const GemvParams &p, hipStream_t s) { return launch("gemv %p m=%u ws=%p cnt=%p", s, p.m, p.ws, p.cnt); }

@@ -215,3 +215,51 @@ print("done")
                          capture_output=True, text=True, timeout=110)
     print(out.stdout, flush=True)
     assert out.returncode == 0 and out.stdout.rstrip().endswith("done"), out.stdout + out.stderr[-2000:]
+
+
+@pytest.mark.parametrize("m", [16, 40])
+def test_wide_values_leave_other_tokens_alone(q, wl, gpu, m):
+    """A wide value shifts its K block for the tokens one launch of the
+    row-split GEMV takes with it (its eight), whose values below 2^-62 lose
+    bits; the rest of its tile keeps theirs."""
+    import torch
+    k, n = 3600, 300
+    w = q.Weight(*wl.gen_weight(7, n, k))
+    rng = np.random.default_rng(m)
+    X = rng.standard_normal((m, k)).astype(np.float32)
+    X[:, 128:256] *= np.float32(2.0 ** -70)      # whole blocks of tiny values
+    X[:, 3456:] *= np.float32(2.0 ** -80)
+    X[0, 130], X[m - 1, 3500] = np.float32(2e30), np.float32(-3e29)
+    X = torch.from_numpy(X).to(gpu)
+    X[1:m - 1, :128], X[1:m - 1, 256:3456] = 0.0, 0.0    # nothing else hides them
+    Y = torch.empty((m, n), device=gpu)
+    q.matmul(w, X, Y)
+    _same_bits(Y, _rows_of_small_calls(q, [w], X, gpu)[0])
+    w.free()
+
+
+def test_wide_products_in_the_mlp(q, wl, gpu):
+    """The same for silu(gate) * up: token 0's products are near 1e30 (column
+    0 of x reaches the norm weight 1e18), the others' near 1e-20, beside a
+    residual of 1e-18."""
+    import torch
+    m, H, I = 24, 1024, 1664
+    w = []
+    for i, (n, k) in enumerate(((I, H), (I, H), (H, I))):
+        W, sc = wl.gen_weight(90 + i, n, k)
+        w.append(q.Weight(W, sc - np.uint16(8 << 7) if i < 2 else sc))   # gate and up times 2^-8
+    nw = np.full(H, -1.0 + 2.0 ** -24, np.float32)
+    nw[0] = 1e18
+    x = np.random.default_rng(3).standard_normal((m, H)).astype(np.float32) * np.float32(1e-18)
+    x[1:, 0], x[0, 0] = 0.0, 5e-18
+    nw, X = torch.from_numpy(nw).to(gpu), torch.from_numpy(x).to(gpu)
+    R, X0 = X.clone(), X.clone()
+    for t in range(0, m, 8):
+        part = R[t:t + 8].clone()
+        q.mlp(*w, nw, part, 0.0)
+        R[t:t + 8] = part
+    q.mlp(*w, nw, X, 0.0)
+    assert torch.isfinite(R).all() and (R[0].abs().max() > 1e26) and not torch.equal(R[8:], X0[8:])
+    _same_bits(X, R)
+    for v in w:
+        v.free()
