@@ -464,7 +464,7 @@ hipError_t launch_gemv_batch(const BatchParams &pin, bool combine, hipStream_t s
     BatchParams p = pin;
     const uint32_t T = p.tile;
     if (p.m == 0 || p.nseg == 0 || p.nseg > 4 || (p.nr != 4 && p.nr != 8) ||
-        !gemv_rows_shape(p.kb, p.nr) || (T != 16 && T != 32))
+        !gemv_rows_shape(p.kb, p.nr) || (T != 16 && T != 32) || (T == 16 && p.m > T))
         return hipErrorInvalidValue;
     p.tiles = (p.m + T - 1) / T;
     p.groups = 0;
@@ -478,9 +478,9 @@ hipError_t launch_gemv_batch(const BatchParams &pin, bool combine, hipStream_t s
     const uint32_t lds = kRing * BatchGeo<16>::kStage + kTabFloats * sizeof(float);
     static_assert(BatchGeo<16>::kStage == BatchGeo<32>::kStage, "one ring size");
     using Kernel = void (*)(BatchParams);
-    static const Kernel kernels[4] = {gemv_batch_kernel<16, false>, gemv_batch_kernel<16, true>,
-                                      gemv_batch_kernel<32, false>, gemv_batch_kernel<32, true>};
-    hipLaunchKernelGGL(kernels[(T == 32 ? 2 : 0) + (p.tiles == 1 ? 1 : 0)], grid, dim3(256), lds, stream, p);
+    const Kernel kernel = T == 16 ? gemv_batch_kernel<16, true>
+                                  : p.tiles == 1 ? gemv_batch_kernel<32, true> : gemv_batch_kernel<32, false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), lds, stream, p);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || !combine) return e;
     hipLaunchKernelGGL((p.nr == 4 ? batch_combine_kernel<4> : batch_combine_kernel<8>),

@@ -165,7 +165,7 @@ struct BatchParams {
     float *ws;           // range sums, segment s at ws_off: [nr][m][nb*128]
     uint32_t m, kb, nseg;
     uint32_t nr;         // K ranges: the row-split GEMV's wavefronts (4 or 8; kPairWaves for gate and up)
-    uint32_t tile;       // tokens per tile (batch_tile), 16 or 32
+    uint32_t tile;       // tokens per tile (batch_tile): 16 (at most 16 tokens) or 32
     uint32_t groups, tiles;   // set by the launch
 };
 uint32_t batch_tile(uint32_t m);                                 // tokens per tile
