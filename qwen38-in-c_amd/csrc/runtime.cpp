@@ -537,18 +537,27 @@ int run_gemv_group(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, cons
 // the launches of eight tokens, which need none and give the same bits.
 constexpr int kNoRoom = -1001;   // internal
 
-// Whether m tokens of row-split weights go as one batch.  From 17 tokens on
-// always: the three launches of a batch replace three or more of the
-// eight-token GEMV (1024 x 1024: 13.5 us either way at 17 tokens, 33.0 ->
-// 13.5 at 63).  9..16 tokens are two such launches, which a batch beats only
-// if each runs long enough: 9 tokens of 3072 -> 1024 11.9 us as two launches,
-// 13.1 as a batch, 4096 -> 1024 14.2 and 12.9, 5120 -> 16480 41.8 and 30.3.
-// kb: the weight's K blocks; of an MLP block (which runs one launch more
-// than its eight-token form, not counting repeats) gate's plus down's: 9
-// tokens of 512 -> 1664 21.0 and 23.2 us, 2048 -> 2048 25.7 and 25.8, 4096
-// -> 4096 36.0 and 34.6, 5120 -> 17408 119.7 and 86.9.
-constexpr uint32_t kBatchMinKb = 28, kBatchMinKbMlp = 33;
-bool batch_pays(uint32_t m, uint32_t kb, uint32_t min_kb) { return m > 2 * kGemvMaxM || (m > kGemvMaxM && kb >= min_kb); }
+// Whether m tokens of row-split weights of nb row groups in all go as one
+// batch.  Times: the eight-token launches, then the batch, us a call.  From
+// 17 tokens on always: the three launches of a batch replace three or more
+// (512 -> 48: 13.9 and 12.7 at 17 tokens, 28.1 and 12.7 at 63; 4096 -> 1024:
+// 23.0 and 14.6, 65.8 and 15.6).  9..16 tokens are two launches, which a
+// batch beats only if each runs long enough: 9 tokens of 3072 -> 1024 12.0
+// and 13.8, 3584 -> 48 12.7 and 13.4, 3584 -> 1024 13.3 and 13.5 (10 tokens
+// 13.5 and 14.0), 3584 -> 2048 13.5 and 13.2, 4096 -> 48 13.2 and 13.4 (16
+// tokens 15.6 and 13.8), 4096 -> 1024 14.2 and 13.2, 5120 -> 16480 40.2 and
+// 28.4.
+constexpr uint32_t kBatchMinKb = 28, kBatchMinNb = 16, kBatchAnyNbKb = 32;
+bool batch_pays(uint32_t m, uint32_t kb, uint64_t nb) {
+    return m > 2 * kGemvMaxM ||
+           (m > kGemvMaxM && (kb >= kBatchAnyNbKb || (kb >= kBatchMinKb && nb >= kBatchMinNb)));
+}
+// An MLP block runs one launch more than its eight-token form, not counting
+// repeats; kb: gate's and down's K blocks together.  9 tokens of 512 -> 1664
+// 21.0 and 22.8 us, 2048 -> 2176 26.6 and 26.6, 512 -> 3712 25.4 and 24.5,
+// 4096 -> 4096 36.2 and 33.0, 5120 -> 17408 119.7 and 81.2.
+constexpr uint32_t kBatchMinKbMlp = 33;
+bool batch_pays_mlp(uint32_t m, uint32_t kb) { return m > 2 * kGemvMaxM || (m > kGemvMaxM && kb >= kBatchMinKbMlp); }
 
 // Whether a call on st may use the batch's scratch.  Not an allocation-free
 // call, whose fixed scratch every stream shares: row-split weights need none
@@ -625,12 +634,11 @@ uint32_t batch_seg(BatchParams &p, uint32_t s, const Weight &w, float *y, const 
     return ws_off + (uint32_t)batch_ws_floats(p.m, w.nb, p.nr);
 }
 
-int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const float *dX, float *const *dY,
-                   hipStream_t st, float *const *resid, Scratch *scr) {
+// nb: row groups of all weights.
+int run_gemv_batch(const q35mm_weight *const *w, uint32_t nseg, uint64_t nb, uint32_t m, const float *dX,
+                   float *const *dY, hipStream_t st, float *const *resid, Scratch *scr) {
     if (!batch_allowed(st, scr)) return kNoRoom;
     const uint32_t cols = w[0]->w.cols, kb = w[0]->w.kb;
-    uint64_t nb = 0;
-    for (uint32_t s = 0; s < nseg; s++) nb += w[s]->w.nb;
     BatchParams p{};
     p.kb = kb;
     p.nseg = nseg;
@@ -671,8 +679,10 @@ int run_gemv(const q35mm_weight *const *w, uint32_t nseg, uint32_t m, const floa
              float *const *dY, hipStream_t st, const GemvInput &in = GemvInput(),
              float *const *resid = nullptr, Scratch *scr = nullptr) {
     const uint32_t cols = w[0]->w.cols;
-    if (batch_pays(m, w[0]->w.kb, kBatchMinKb) && in.xmode == kXPlain && uses_gemv_rows(w[0]->w)) {   // same K: one kind
-        const int rc = run_gemv_batch(w, nseg, m, dX, dY, st, resid, scr);
+    uint64_t nb = 0;
+    for (uint32_t s = 0; s < nseg; s++) nb += w[s]->w.nb;
+    if (batch_pays(m, w[0]->w.kb, nb) && in.xmode == kXPlain && uses_gemv_rows(w[0]->w)) {   // same K: one kind
+        const int rc = run_gemv_batch(w, nseg, nb, m, dX, dY, st, resid, scr);
         if (rc != kNoRoom) return rc;
     }
     for (uint32_t t0 = 0; t0 < m; t0 += kGemvMaxM) {
@@ -1926,7 +1936,7 @@ Q35MM_API int q35mm_mlp(const q35mm_weight *gate, const q35mm_weight *up, const 
             // residual add.
             const bool norm_in = m == 1 && H <= kPairNormMaxCols && g_dev.mlp_pair == 1;
             if (!norm_in) HIP_TRY(launch_rmsnorm(dX, H, dNormW, xn, H, m, H, eps, st));
-            if (batch_pays(m, gate->w.kb + down->w.kb, kBatchMinKbMlp) && uses_gemv_rows(down->w)) {
+            if (batch_pays_mlp(m, gate->w.kb + down->w.kb) && uses_gemv_rows(down->w)) {
                 rc = run_mlp_batch(gate, up, down, m, xn, dX, st);
                 if (rc != kNoRoom) return rc;
             }

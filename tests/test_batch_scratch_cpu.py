@@ -249,3 +249,21 @@ def test_mlp_ranges_are_the_paired_kernels(stub_path, monkeypatch, waves):
     lb.lib.q35mm_shutdown()
     assert seen[8] == [("pair", "4"), ("rows", str(waves))]
     assert seen[24] == [("batch", "4"), ("batch_swiglu", "4"), ("batch", str(waves))]
+
+
+@pytest.mark.parametrize("m,cols,rows,batch", [
+    (8, 5120, 2048, False), (9, 4096, 48, True), (16, 3968, 1920, False), (9, 3968, 1921, True),
+    (9, 3457, 1921, True), (16, 3456, 20000, False), (17, 512, 48, True)])
+def test_which_sizes_are_batched(lib, m, cols, rows, batch):
+    """From 17 tokens on every row-split weight; 9..16 tokens from 32 K
+    blocks on, from 28 on with 16 row groups."""
+    rc, rec = lib.matmul(lib.weight(rows, cols), m, S)
+    assert rc == 0 and ("batch" in kinds(rec)) == batch
+
+
+@pytest.mark.parametrize("rows,batch", [((1000, 896), False), ((1000, 1000), True)])
+def test_row_groups_of_all_weights_count(lib, rows, batch):
+    ws = (C.c_void_p * 2)(*[lib.weight(n, 3584).value for n in rows])
+    ys = (C.c_void_p * 2)(lib.y, lib.y)
+    assert lib.lib.q35mm_matmul_multi(ws, 2, 9, lib.x, ys, S) == 0
+    assert ("batch" in kinds(lib.take())) == batch

@@ -36,11 +36,12 @@ def _same_bits(a, b):
     assert torch.equal(a.view(torch.int32), b.view(torch.int32))
 
 
-# 9..16 tokens: 28 K blocks or more (fewer go as two small calls)
+# 9..16 tokens: 32 K blocks or more, or 28 with 16 row groups (fewer go as two small calls)
 @pytest.mark.parametrize("m,k,rows", [(9, 3600, (200,)), (16, 4571, (4100,)), (12, 5120, (1300, 48, 5000)),
                                       (10, 20480, (1,)), (17, 5120, (1024,)), (32, 640, (33000,)), (18, 400, (70,)),
                                       (33, 20480, (129,)), (63, 17400, (300,)), (24, 1032, (130, 48, 1, 5000)),
-                                      (63, 768, (16300, 70)), (16, 3456, (300,)), (9, 3457, (300,))])
+                                      (63, 768, (16300, 70)), (16, 3456, (300,)), (9, 3457, (300,)),
+                                      (9, 4200, (200,)), (13, 3457, (2100,)), (16, 3968, (1000, 1000))])
 def test_batch_rows_are_small_calls_bitwise(q, wl, gpu, m, k, rows):
     import torch
     ws = [q.Weight(*wl.gen_weight_ragged(k + i, n, k)) for i, n in enumerate(rows)]
@@ -65,7 +66,7 @@ def test_batch_rows_are_small_calls_bitwise(q, wl, gpu, m, k, rows):
 def test_batch_wide_values(q, wl, gpu, m):
     """Blocks holding values past 2^96 or infinities are staged shifted."""
     import torch
-    k, n = 3600, 300
+    k, n = 4200, 300
     w = q.Weight(*wl.gen_weight(5, n, k))
     X = wl.gen_act(6, m, k)
     X[0, 3], X[1, 700], X[2, 999] = np.inf, -np.inf, np.float32(3.4e38)
@@ -188,7 +189,7 @@ import q35mm as q, workload as wl
 gpu = torch.device("cuda:0")
 def same(a, b):
     assert torch.equal(a.view(torch.int32), b.view(torch.int32))
-for m, k, n in ((9, 3600, 200), (24, 1032, 300), (63, 5120, 129)):
+for m, k, n in ((9, 4200, 200), (24, 1032, 300), (63, 5120, 129)):
     print("matmul", m, k, n, flush=True)
     w = q.Weight(*wl.gen_weight(k, n, k))
     X = torch.from_numpy(wl.gen_act(m, m, k)).to(gpu)
@@ -223,12 +224,12 @@ def test_wide_values_leave_other_tokens_alone(q, wl, gpu, m):
     row-split GEMV takes with it (its eight), whose values below 2^-62 lose
     bits; the rest of its tile keeps theirs."""
     import torch
-    k, n = 3600, 300
+    k, n = 4200, 300
     w = q.Weight(*wl.gen_weight(7, n, k))
     rng = np.random.default_rng(m)
     X = rng.standard_normal((m, k)).astype(np.float32)
     X[:, 128:256] *= np.float32(2.0 ** -70)      # whole blocks of tiny values
-    X[:, 3456:] *= np.float32(2.0 ** -80)
+    X[:, 3456:] *= np.float32(2.0 ** -80)        # the last, partial block too
     X[0, 130], X[m - 1, 3500] = np.float32(2e30), np.float32(-3e29)
     X = torch.from_numpy(X).to(gpu)
     X[1:m - 1, :128], X[1:m - 1, 256:3456] = 0.0, 0.0    # nothing else hides them
