@@ -68,8 +68,12 @@ int q35mm_weight_shape(const q35mm_weight *w, uint32_t *rows, uint32_t *cols);
 size_t q35mm_weight_bytes(const q35mm_weight *w);
 
 /* Y[t][r] for t < m, X [m][cols] fp32, Y [m][rows] fp32, device pointers.
- * Dispatch by m: m <= 8 -> decode GEMV; 8 < m < Q35MM_GEMM_MIN_M -> decode
- * GEMV over groups of 8 tokens; m >= Q35MM_GEMM_MIN_M -> bf16 MFMA GEMM. */
+ * Dispatch by m: m <= 8 -> decode GEMV; 8 < m < Q35MM_GEMM_MIN_M -> of
+ * weights of 4..160 K blocks of 128 columns one pass over the weight for up
+ * to 32 tokens where that is faster, else the decode GEMV over groups of 8
+ * tokens, the same bits; m >= Q35MM_GEMM_MIN_M -> bf16 MFMA GEMM.  The pass
+ * keeps scratch per stream (up to 4 * m * rows fp32); a graph capture, a
+ * call without memory for it or on hipStreamPerThread takes groups of 8. */
 int q35mm_matmul(const q35mm_weight *w, uint32_t m, const float *dX, float *dY,
                  void *stream);
 /* q35mm_matmul without any allocation.  No counterpart in the reference:
@@ -92,7 +96,7 @@ int q35mm_matmul(const q35mm_weight *w, uint32_t m, const float *dX, float *dY,
  * kernels overlap on one device (different streams) race. */
 int q35mm_matmul_noalloc(const q35mm_weight *w, uint32_t m, const float *dX,
                          float *dY, void *stream);
-/* Decode GEMV for any m (groups of 8 tokens), fp32-accurate. */
+/* q35mm_matmul's dispatch below Q35MM_GEMM_MIN_M for any m, fp32-accurate. */
 int q35mm_gemv(const q35mm_weight *w, uint32_t m, const float *dX, float *dY,
                void *stream);
 /* Prefill GEMM for any m: activations rounded to bf16, bf16 MFMA with fp32

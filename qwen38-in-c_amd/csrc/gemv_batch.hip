@@ -34,8 +34,8 @@
 // is bound by each wavefront's chain of 34 K blocks.
 //
 // Whole calls against the row-split GEMV in groups of eight, us: 5120 ->
-// 16480 at 24 tokens 66.8 -> 36.8, at 63 tokens 178.8 -> 51.5; 17408 -> 5120
-// 77.5 -> 37.5 and 207.8 -> 56.0.  (The runtime's batch_pays says from which
+// 16480 at 24 tokens 66.3 -> 36.6, at 63 tokens 176.9 -> 50.9; 17408 -> 5120
+// 77.5 -> 38.0 and 207.8 -> 55.4.  (The runtime's batch_pays says from which
 // sizes on it is taken.)
 //
 // Bits.  The decode GEMV sums each of its K ranges block by block (one fmaf

@@ -4,9 +4,10 @@ weight in one pass over it, below the prefill GEMM.
 Its sums are the row-split GEMV's, so every row of a batch is, bit for bit,
 the row of a call of one to eight tokens (which the other tests hold against
 the oracle): edges of the token tiles (16 and 32), 4..160 K blocks (a last
-turn of the three-deep ring of each length), partial blocks both ways, both
-work splits (few and many row groups), several weights, values of any
-magnitude.
+turn of the four-deep ring of each length), partial blocks both ways, four
+and eight K ranges, one row group to hundreds, several weights, values of
+any magnitude.  Which calls are batched, and on what scratch, is
+test_batch_scratch_cpu.py's.
 """
 import os
 import subprocess
@@ -115,8 +116,9 @@ def test_batch_beyond_the_gemm(q, wl, gpu):
 
 
 def test_batch_capture(q, wl, gpu):
-    """A capture on a stream that has no scratch yet and one after a call of
-    the same size on that stream both replay to the eager bits."""
+    """Captures run eight tokens a launch, on a stream the library has not
+    seen and on one that ran the same call as a batch: both replay to the
+    eager bits (test_batch_scratch_cpu.py sees the launches)."""
     import torch
     w = q.Weight(*wl.gen_weight(12, 700, 1024))
     X = torch.from_numpy(wl.gen_act(13, 24, 1024)).to(gpu)
