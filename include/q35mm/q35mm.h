@@ -72,8 +72,9 @@ size_t q35mm_weight_bytes(const q35mm_weight *w);
  * weights of 4..160 K blocks of 128 columns one pass over the weight for up
  * to 32 tokens where that is faster, else the decode GEMV over groups of 8
  * tokens, the same bits; m >= Q35MM_GEMM_MIN_M -> bf16 MFMA GEMM.  The pass
- * keeps scratch per stream (up to 4 * m * rows fp32); a graph capture, a
- * call without memory for it or on hipStreamPerThread takes groups of 8. */
+ * keeps scratch per stream (up to 4 * m * rows fp32, 4 GiB over all streams,
+ * given back by q35mm_stream_release); a graph capture, a call without
+ * memory for it or on hipStreamPerThread takes groups of 8. */
 int q35mm_matmul(const q35mm_weight *w, uint32_t m, const float *dX, float *dY,
                  void *stream);
 /* q35mm_matmul without any allocation.  No counterpart in the reference:

@@ -112,7 +112,11 @@ struct Scratch {
 struct BatchBuf {
     DevBuf buf;
     std::vector<void *> old;
+    size_t bytes = 0;   // of all of them
 };
+// Of all streams together.  A stream destroyed without a release keeps its
+// buffer, as it keeps its scratch set; matmuls of 9..63 tokens kept nothing.
+constexpr size_t kBatchMaxBytes = (size_t)4 << 30;
 
 struct Device {
     int id = -1;
@@ -124,6 +128,7 @@ struct Device {
     // eager calls), and a stream that only ran batches has no set a capture
     // could be given.
     std::unordered_map<hipStream_t, BatchBuf> batch;
+    size_t batch_bytes = 0;
     std::vector<void *> retired;       // buffers a captured graph may still use (freed at shutdown)
     DevBuf dx, dy;    // activation staging for the host-pointer ABI
     void *up_pin[4] = {};        // pinned chunks of the file -> HBM upload ring
@@ -587,10 +592,11 @@ int batch_scratch(hipStream_t st, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t
         // No wait for the device, as these calls never had one, and no
         // failure: eight tokens need no memory.  The relaxed mode lets the
         // thread allocate while another thread captures.
+        const size_t cap = (std::max(xb + wb, 2 * b.cap) + 4095) & ~(size_t)4095;
+        if (g_dev.batch_bytes + cap > kBatchMaxBytes) return kNoRoom;
         hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
         HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
         void *ptr = nullptr;
-        const size_t cap = (std::max(xb + wb, 2 * b.cap) + 4095) & ~(size_t)4095;
         const hipError_t e = hipMalloc(&ptr, cap);
         HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
         if (e != hipSuccess) {
@@ -600,6 +606,8 @@ int batch_scratch(hipStream_t st, uint32_t mp, uint32_t kb, uint32_t nb, uint8_t
         if (b.ptr) bb.old.push_back(b.ptr);
         b.ptr = ptr;
         b.cap = cap;
+        bb.bytes += cap;
+        g_dev.batch_bytes += cap;
     }
     *xs = static_cast<uint8_t *>(b.ptr);
     *xf = reinterpret_cast<float *>(*xs + ab);
@@ -615,6 +623,7 @@ hipError_t free_batch(BatchBuf &b) {
         const hipError_t f = ptr ? hipFree(ptr) : hipSuccess;
         if (e == hipSuccess) e = f;
     }
+    g_dev.batch_bytes -= b.bytes;
     b = BatchBuf();
     return e;
 }

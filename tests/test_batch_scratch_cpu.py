@@ -267,3 +267,26 @@ def test_row_groups_of_all_weights_count(lib, rows, batch):
     ys = (C.c_void_p * 2)(lib.y, lib.y)
     assert lib.lib.q35mm_matmul_multi(ws, 2, 9, lib.x, ys, S) == 0
     assert ("batch" in kinds(lib.take())) == batch
+
+
+def test_scratch_of_all_streams_is_bounded(lib):
+    """Streams that come and go without a release: the batch's scratch stays
+    within its bound, later streams run eight tokens a launch, and a released
+    stream's share serves another."""
+    w = lib.weight(60000, 512)               # 62 MB of range sums at 63 tokens
+    total = 0
+    for i in range(100):
+        st = 0x100000 + 16 * i
+        rc, rec = lib.matmul(w, 63, st)
+        assert rc == 0
+        total += sum(int(ln.split()[2]) for k, _, ln in rec if k == "malloc")
+        if "batch" in kinds(rec):
+            first_without = i + 1
+    assert total <= 4 << 30 and 40 < first_without < 100
+    rc, rec = lib.matmul(w, 63, 0x100000 + 16 * 99)
+    assert rc == 0 and kinds(rec) == ["rows"] * 8
+    assert lib.lib.q35mm_stream_release(0x100000) == 0
+    rc, rec = lib.matmul(w, 63, 0x100000 + 16 * 99)
+    assert rc == 0 and "batch" in kinds(rec)
+    for i in range(100):
+        assert lib.lib.q35mm_stream_release(0x100000 + 16 * i) == 0
