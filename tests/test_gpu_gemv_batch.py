@@ -266,3 +266,29 @@ def test_wide_products_in_the_mlp(q, wl, gpu):
     _same_bits(X, R)
     for v in w:
         v.free()
+
+
+def test_first_batch_beside_a_capture(q, wl, gpu):
+    """A batch whose scratch is allocated while another stream is captured:
+    the call works and the capture stays valid."""
+    import torch
+    w = q.Weight(*wl.gen_weight(16, 700, 5120))
+    X = torch.from_numpy(wl.gen_act(17, 24, 5120)).to(gpu)
+    want = _rows_of_small_calls(q, [w], X, gpu)[0]
+    Y, Z = torch.zeros_like(want), torch.zeros_like(want)
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    q.stream_release(t.cuda_stream)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        q.matmul(w, X, Y)
+        q.matmul(w, X, Z, stream=t.cuda_stream)
+    torch.cuda.synchronize()
+    _same_bits(Z, want)
+    for _ in range(3):
+        Y.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        _same_bits(Y, want)
+    w.free()
